@@ -8,7 +8,8 @@
 //     1 KiB of a row and every x chunk serves all rows of the group.
 //   * gemv_valu (M <= 4, longer rows): one wave per R weight rows streaming
 //     16-byte chunks in a loop.
-//   * linear_mfma (M > 4): v_mfma_f32_16x16x32_bf16 on 16-row weight tiles
+//   * linear_mt (M > 16, linear_mt.hip): up to 64 batch rows per read of W.
+//   * linear_mfma (4 < M <= 16): v_mfma_f32_16x16x32_bf16 on 16-row weight tiles
 //     against 16 batch rows; the K range is split over the 4 waves of a
 //     block and the partial tiles are summed through LDS.
 // They fuse the RMSNorm prologue (M <= 4: statistics from the x chunks in
@@ -1064,29 +1065,28 @@ void launch_mfma(const LinearArgs& a, hipStream_t s) {
   }
 }
 
-// The batched stages with the RMSNorm prologue (M > 4, K = 4096: four
+// The batched stages with the RMSNorm prologue (4 < M <= 16, K = 4096: four
 // 256-wide chunks per wave) run the X-stationary kernel, which normalises in
 // its prologue: gate/up with 2 or 3 tiles per CU as multi-tile blocks, the
 // 24-row blocks of a QKV-sized projection, and up to one 16-row tile per CU.
 // Larger shapes (an LM head) keep the staging pass and the streaming blocks.
 bool launch_xs_norm(const LinearArgs& a, hipStream_t s) {
-  if (a.K != 4 * 4 * kMfmaKC || a.x_packed) return false;
+  if (a.M > 16 || a.K != 4 * 4 * kMfmaKC || a.x_packed) return false;
   const int64_t cus = num_cus(), tx = (a.N + 15) / 16;
-  const unsigned gy = unsigned((a.M + 15) / 16);
   const dim3 block(4 * kWave);
   if (a.epi == kEpiSilu) {
-    if (tx == 3 * cus) hipLaunchKernelGGL((linear_xs_kernel<2, true, 4, 3, 0, true>), dim3(unsigned(cus), gy), block, 0, s, a);
-    else if (tx == 2 * cus) hipLaunchKernelGGL((linear_xs_kernel<2, true, 4, 2, 0, true>), dim3(unsigned(cus), gy), block, 0, s, a);
-    else if (tx * gy <= cus) hipLaunchKernelGGL((linear_xs_kernel<2, true, 4, 1, 0, true>), dim3(unsigned(tx), gy), block, 0, s, a);
+    if (tx == 3 * cus) hipLaunchKernelGGL((linear_xs_kernel<2, true, 4, 3, 0, true>), dim3(unsigned(cus)), block, 0, s, a);
+    else if (tx == 2 * cus) hipLaunchKernelGGL((linear_xs_kernel<2, true, 4, 2, 0, true>), dim3(unsigned(cus)), block, 0, s, a);
+    else if (tx <= cus) hipLaunchKernelGGL((linear_xs_kernel<2, true, 4, 1, 0, true>), dim3(unsigned(tx)), block, 0, s, a);
     else return false;
     return true;
   }
-  if (a.M <= 16 && a.N > 16 * cus && a.N <= 24 * cus) {
+  if (a.N > 16 * cus && a.N <= 24 * cus) {
     hipLaunchKernelGGL((linear_xs_kernel<2, false, 4, 1, 8, true>), dim3(unsigned((a.N + 23) / 24)), block, 0, s, a);
     return true;
   }
-  if (tx * gy <= cus) {
-    hipLaunchKernelGGL((linear_xs_kernel<1, false, 4, 1, 0, true>), dim3(unsigned(tx), gy), block, 0, s, a);
+  if (tx <= cus) {
+    hipLaunchKernelGGL((linear_xs_kernel<1, false, 4, 1, 0, true>), dim3(unsigned(tx)), block, 0, s, a);
     return true;
   }
   return false;
@@ -1124,8 +1124,8 @@ int launch_linear(const LinearArgs& a, hipStream_t s) {
       silu ? launch_valu_m<false, true>(a, s) : launch_valu_m<false, false>(a, s);
     }
   } else {
-    // M > 4 with the RMSNorm prologue: the X-stationary kernel normalises in
-    // its prologue where the shape allows (one block per CU: every block
+    // 4 < M <= 16 with the RMSNorm prologue: the X-stationary kernel normalises
+    // in its prologue where the shape allows (one block per CU: every block
     // loads X once anyway); otherwise the input is staged once as
     // bf16(x * rsqrt(mean x^2 + eps) * w) (the reference's staging) into the
     // caller's workspace and a plain MFMA GEMM runs on it (normalising inside
@@ -1149,7 +1149,8 @@ int launch_linear(const LinearArgs& a, hipStream_t s) {
       b.ldx = a.K;
       b.norm = 0;
     }
-    silu ? launch_mfma<true>(b, s) : launch_mfma<false>(b, s);
+    if (linear_mt_supported(b)) launch_linear_mt(b, s);
+    else silu ? launch_mfma<true>(b, s) : launch_mfma<false>(b, s);
   }
   return launch_status("linear");
 }

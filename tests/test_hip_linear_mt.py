@@ -1,0 +1,64 @@
+"""Linear stages of 17 and more batch rows (one read of W per 64 rows) against the oracle.
+
+Sizes at the edges of the kernel: batch blocks of 16 (2, 3 or 4 per block,
+two 64-row groups), weight-row remainders of a 16-row tile, K with fewer
+chunks than waves and a masked last chunk, one tile per CU / two blocks per
+CU / two-tile blocks.  Bar: bf16 allclose(atol 2e-2, rtol 1e-2) against the
+fp32-accumulated oracle, as for the other linear stages.
+"""
+
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from ezops import _hip
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def g(a):
+    return torch.from_numpy(np.ascontiguousarray(a)).to(torch.bfloat16).to(DEV)
+
+
+def _run(M, N, K, epi, norm, pad=0, seed=0):
+    rng = np.random.default_rng(seed)
+    bf = lambda *s: oracle.bf16(rng.standard_normal(s, dtype=np.float32))  # noqa: E731
+    X, R = bf(M, K + pad), bf(M, N)
+    W, W2 = bf(N, K) * np.float32(2.0 ** -6), bf(N, K) * np.float32(2.0 ** -6)  # exact in bf16
+    w = oracle.bf16(rng.standard_normal(K).astype(np.float32) * 0.1 + 1)
+    Xn = oracle.rmsnorm_bf16(X[:, :K], w) if norm else X[:, :K]
+    ref = oracle.linear_bf16(Xn, W)
+    if epi == 1:
+        ref = oracle.bf16(R + ref)
+    elif epi == 2:
+        u = oracle.linear_bf16(Xn, W2)
+        ref = oracle.bf16(oracle.bf16(ref / (1 + np.exp(-ref.astype(np.float64)))) * u)
+    elif epi == 3:
+        ref = Xn @ W.T
+    tX, tW, tW2, tR, tw = g(X), g(W), g(W2), g(R), g(w)
+    # a guard row behind Y: nothing is written past row M
+    Y = torch.full((M + 1, N), 7.0, dtype=torch.float32 if epi == 3 else torch.bfloat16, device=DEV)
+    ws = torch.zeros(max(256, _hip.size("ezops_linear_stage_workspace_size", M, K, norm)), dtype=torch.uint8, device=DEV)
+    _hip.call("ezops_linear_stage_bf16", tX.data_ptr(), K + pad, tW.data_ptr(), tW2.data_ptr(), Y.data_ptr(), N,
+              tR.data_ptr(), N, tw.data_ptr(), norm, 1e-6, epi, M, N, K, ws.data_ptr(), ws.numel(), _hip.stream())
+    torch.cuda.synchronize()
+    out = Y.float().cpu().numpy()
+    assert (out[M] == 7.0).all()
+    np.testing.assert_allclose(out[:M], ref, rtol=1e-2, atol=2e-2)
+
+
+@pytest.mark.parametrize("M", [17, 32, 33, 48, 49, 64, 65, 100])
+@pytest.mark.parametrize("epi,norm", [(0, 0), (1, 0), (2, 1), (3, 0)])
+@pytest.mark.parametrize("N,K", [(48, 512), (37, 1032), (16, 40), (250, 2048)])
+def test_linear_mt_edges(M, epi, norm, N, K):
+    _run(M, N, K, epi, norm, pad=0 if norm else 8 * (N % 2))
+
+
+# 4104 rows: two blocks per CU and a remainder; 16400: two-tile blocks, odd
+# tile count; 4096 x 4096: one tile per CU.
+@pytest.mark.parametrize("M,N,K,epi,norm", [(33, 4104, 256, 1, 0), (64, 16400, 512, 0, 1), (20, 16424, 256, 3, 0),
+                                            (64, 4096, 4096, 1, 0), (40, 4112, 1024, 2, 1)])
+def test_linear_mt_tilings(M, N, K, epi, norm):
+    _run(M, N, K, epi, norm, seed=1)
