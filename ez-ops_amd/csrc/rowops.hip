@@ -2,9 +2,9 @@
 // the STREAM probes used to measure the HBM peak.
 //
 // Row ops keep the whole row in registers (one HBM read, one write): a block
-// of BS threads holds VPT float4 per thread.  Rows longer than the register
-// budget, or rows that are not 16-byte aligned, take a looped kernel that
-// re-reads the row.
+// of BS threads holds VPT float4 per thread, at any row alignment.  Longer
+// softmax rows are cut into chunks over two launches; longer RMSNorm rows take
+// a looped kernel that re-reads the row.
 #include "common.h"
 #include "internal.h"
 #include "prof.h"
@@ -20,6 +20,22 @@ constexpr float kLog2e = 1.4426950408889634f;
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
+// 16-byte accesses of rows that start at any element: gfx950 takes global
+// loads and stores at every byte address (the HSA runtime's unaligned access
+// mode), so rows of odd length keep the wide accesses; only the last dim % 4
+// (% 8) elements are scalar.  Rows that were not 16-byte aligned took a looped
+// scalar kernel before: softmax 4000 x 32767 434 -> 198 us, RMSNorm 8000 x 4097
+// bf16 70 -> 33, fp32 83 -> 52.
+typedef float f32x4u_t __attribute__((ext_vector_type(4), aligned(4)));
+typedef unsigned int u32x4u_t __attribute__((ext_vector_type(4), aligned(2)));
+__device__ __forceinline__ float4 ld4u(const float* p) {
+  const f32x4u_t v = *reinterpret_cast<const f32x4u_t*>(p);
+  return make_float4(v.x, v.y, v.z, v.w);
+}
+__device__ __forceinline__ void st4u(float* p, const float4& v) {
+  *reinterpret_cast<f32x4u_t*>(p) = f32x4u_t{v.x, v.y, v.z, v.w};
+}
+
 // ---------------------------------------------------------------- RMSNorm f32
 template <int BS, int VPT>
 __global__ __launch_bounds__(BS) void rmsnorm_f32_reg_kernel(const float* __restrict__ X,
@@ -27,17 +43,17 @@ __global__ __launch_bounds__(BS) void rmsnorm_f32_reg_kernel(const float* __rest
                                                               int64_t dim, float eps) {
   EZ_PROF_WAVE(kProfRmsnormF32);
   __shared__ float red[BS / kWave];
-  const int64_t row = blockIdx.x;
-  const float4* x = reinterpret_cast<const float4*>(X + row * dim);
-  float4* o = reinterpret_cast<float4*>(Out + row * dim);
-  const int64_t n4 = dim >> 2;
+  const float* x = X + int64_t(blockIdx.x) * dim;
+  float* o = Out + int64_t(blockIdx.x) * dim;
+  const int64_t n4 = dim >> 2, ti = 4 * n4 + threadIdx.x;  // ti: the last dim % 4 elements
   float4 v[VPT];
-  float ss = 0.f;
 #pragma unroll
   for (int j = 0; j < VPT; ++j) {
     const int64_t c = threadIdx.x + int64_t(j) * BS;
-    v[j] = c < n4 ? x[c] : make_float4(0.f, 0.f, 0.f, 0.f);
+    v[j] = c < n4 ? ld4u(x + 4 * c) : make_float4(0.f, 0.f, 0.f, 0.f);
   }
+  const float vt = ti < dim ? x[ti] : 0.f;
+  float ss = vt * vt;
 #pragma unroll
   for (int j = 0; j < VPT; ++j) ss += v[j].x * v[j].x + v[j].y * v[j].y + v[j].z * v[j].z + v[j].w * v[j].w;
   ss = block_reduce<BS / kWave, false>(ss, red);
@@ -45,8 +61,9 @@ __global__ __launch_bounds__(BS) void rmsnorm_f32_reg_kernel(const float* __rest
 #pragma unroll
   for (int j = 0; j < VPT; ++j) {
     const int64_t c = threadIdx.x + int64_t(j) * BS;
-    if (c < n4) o[c] = make_float4(v[j].x * r, v[j].y * r, v[j].z * r, v[j].w * r);
+    if (c < n4) st4u(o + 4 * c, make_float4(v[j].x * r, v[j].y * r, v[j].z * r, v[j].w * r));
   }
+  if (ti < dim) o[ti] = vt * r;
 }
 
 __global__ __launch_bounds__(256) void rmsnorm_f32_loop_kernel(const float* __restrict__ X,
@@ -64,8 +81,9 @@ __global__ __launch_bounds__(256) void rmsnorm_f32_loop_kernel(const float* __re
 }
 
 // ------------------------------------------------------ RMSNorm bf16 + weight
-// One block per row; VPT chunks of 8 bf16 per thread.  PACKED writes the
-// row into the MFMA-packed layout of the skinny GEMM (dim % 32 == 0).
+// One block per row; VPT chunks of 8 bf16 per thread, the last dim % 8
+// elements one to a thread.  PACKED writes the row into the MFMA-packed layout
+// of the skinny GEMM (dim % 32 == 0).
 template <int BS, int VPT, bool PACKED = false>
 __global__ __launch_bounds__(BS) void rmsnorm_bf16_reg_kernel(const uint16_t* __restrict__ X,
                                                                const uint16_t* __restrict__ W,
@@ -74,28 +92,29 @@ __global__ __launch_bounds__(BS) void rmsnorm_bf16_reg_kernel(const uint16_t* __
   EZ_PROF_WAVE(kProfRmsnormBf16);
   __shared__ float red[BS / kWave];
   const int64_t row = blockIdx.x;
-  const uint4* x = reinterpret_cast<const uint4*>(X + row * dim);
-  const uint4* w = reinterpret_cast<const uint4*>(W);
-  uint4* o = reinterpret_cast<uint4*>(Out + row * dim);  // row-major output
-  const int64_t n8 = dim >> 3;
-  uint4 v[VPT], wv[VPT];
-  float ss = 0.f;
+  const uint16_t* x = X + row * dim;
+  uint16_t* o = Out + row * dim;  // row-major output
+  const int64_t n8 = dim >> 3, ti = 8 * n8 + threadIdx.x;
+  u32x4u_t v[VPT], wv[VPT];
 #pragma unroll
   for (int j = 0; j < VPT; ++j) {
     const int64_t c = threadIdx.x + int64_t(j) * BS;
-    v[j] = c < n8 ? x[c] : make_uint4(0, 0, 0, 0);
+    v[j] = c < n8 ? *reinterpret_cast<const u32x4u_t*>(x + 8 * c) : u32x4u_t{0u, 0u, 0u, 0u};
   }
   // The weight pieces are requested with the row, not after the reduction.
   constexpr uint32_t one2 = 0x3f803f80u;  // two bf16 1.0
 #pragma unroll
   for (int j = 0; j < VPT; ++j) {
     const int64_t c = threadIdx.x + int64_t(j) * BS;
-    wv[j] = (W && c < n8) ? w[c] : make_uint4(one2, one2, one2, one2);
+    wv[j] = (W && c < n8) ? *reinterpret_cast<const u32x4u_t*>(W + 8 * c) : u32x4u_t{one2, one2, one2, one2};
   }
+  const bool own_t = !PACKED && ti < dim;
+  const float vt = own_t ? bf2f(x[ti]) : 0.f, wt = own_t && W ? bf2f(W[ti]) : 1.f;
+  float ss = vt * vt;
 #pragma unroll
   for (int j = 0; j < VPT; ++j) {
     float f[8];
-    unpack8(v[j], f);
+    unpack8(make_uint4(v[j].x, v[j].y, v[j].z, v[j].w), f);
 #pragma unroll
     for (int e = 0; e < 8; ++e) ss = fmaf(f[e], f[e], ss);
   }
@@ -106,14 +125,15 @@ __global__ __launch_bounds__(BS) void rmsnorm_bf16_reg_kernel(const uint16_t* __
     const int64_t c = threadIdx.x + int64_t(j) * BS;
     if (c < n8) {
       float f[8], g[8];
-      unpack8(v[j], f);
-      unpack8(wv[j], g);
+      unpack8(make_uint4(v[j].x, v[j].y, v[j].z, v[j].w), f);
+      unpack8(make_uint4(wv[j].x, wv[j].y, wv[j].z, wv[j].w), g);
       const uint4 y = make_uint4(pack_bf2(f[0] * r * g[0], f[1] * r * g[1]), pack_bf2(f[2] * r * g[2], f[3] * r * g[3]),
                                  pack_bf2(f[4] * r * g[4], f[5] * r * g[5]), pack_bf2(f[6] * r * g[6], f[7] * r * g[7]));
       if constexpr (PACKED) *reinterpret_cast<uint4*>(Out + packed_index(row, 8 * c, dim)) = y;
-      else o[c] = y;
+      else *reinterpret_cast<u32x4u_t*>(o + 8 * c) = u32x4u_t{y.x, y.y, y.z, y.w};
     }
   }
+  if (own_t) o[ti] = f2bf(vt * r * wt);
 }
 
 __global__ __launch_bounds__(256) void rmsnorm_bf16_loop_kernel(const uint16_t* __restrict__ X,
@@ -136,27 +156,30 @@ __global__ __launch_bounds__(256) void rmsnorm_bf16_loop_kernel(const uint16_t* 
 }
 
 // ------------------------------------------------------------------ softmax
+// A block per row, the row in registers (dim <= 4 * BS * VPT): one read, one
+// write.  The last dim % 4 elements sit in the first threads.
 template <int BS, int VPT>
 __global__ __launch_bounds__(BS) void softmax_reg_kernel(const float* __restrict__ X,
                                                           float* __restrict__ Out, int64_t dim) {
   EZ_PROF_WAVE(kProfSoftmax);
   __shared__ float red[BS / kWave];
-  const int64_t row = blockIdx.x;
-  const float4* x = reinterpret_cast<const float4*>(X + row * dim);
-  float4* o = reinterpret_cast<float4*>(Out + row * dim);
-  const int64_t n4 = dim >> 2;
+  const float* x = X + int64_t(blockIdx.x) * dim;
+  float* o = Out + int64_t(blockIdx.x) * dim;
+  const int64_t n4 = dim >> 2, ti = 4 * n4 + threadIdx.x;
   float4 v[VPT];
   float mx = -INFINITY;
 #pragma unroll
   for (int j = 0; j < VPT; ++j) {
     const int64_t c = threadIdx.x + int64_t(j) * BS;
-    v[j] = c < n4 ? x[c] : make_float4(-INFINITY, -INFINITY, -INFINITY, -INFINITY);
+    v[j] = c < n4 ? ld4u(x + 4 * c) : make_float4(-INFINITY, -INFINITY, -INFINITY, -INFINITY);
   }
+  float vt = ti < dim ? x[ti] : -INFINITY;
 #pragma unroll
   for (int j = 0; j < VPT; ++j) mx = fmaxf(mx, fmaxf(fmaxf(v[j].x, v[j].y), fmaxf(v[j].z, v[j].w)));
-  mx = block_reduce<BS / kWave, true>(mx, red);
+  mx = block_reduce<BS / kWave, true>(fmaxf(mx, vt), red);
   const float mb = mx * kLog2e;
-  float sum = 0.f;
+  vt = exp2f(fmaf(vt, kLog2e, -mb));
+  float sum = vt;
 #pragma unroll
   for (int j = 0; j < VPT; ++j) {
     v[j].x = exp2f(fmaf(v[j].x, kLog2e, -mb));
@@ -170,12 +193,102 @@ __global__ __launch_bounds__(BS) void softmax_reg_kernel(const float* __restrict
 #pragma unroll
   for (int j = 0; j < VPT; ++j) {
     const int64_t c = threadIdx.x + int64_t(j) * BS;
-    if (c < n4) o[c] = make_float4(v[j].x * inv, v[j].y * inv, v[j].z * inv, v[j].w * inv);
+    if (c < n4) st4u(o + 4 * c, make_float4(v[j].x * inv, v[j].y * inv, v[j].z * inv, v[j].w * inv));
+  }
+  if (ti < dim) o[ti] = vt * inv;
+}
+
+// Rows too long for one block's registers, cut into C chunks of `per` floats
+// (<= 4 kSplitBS kSplitVPT; 2 C <= every chunk) over two launches, so that a
+// few long rows fill the chip.  The first writes each chunk's (maximum in
+// log2 units, sum of exponentials) to every chunk's place in Out -- chunk k
+// holds the row's C pairs in its first 2 C floats -- and the second reads its
+// chunk's copy, merges the pairs and overwrites the chunk.  Each block of the
+// second touches its own chunk alone, so no block waits for another; the
+// launch boundary orders the two.  X is read twice (the second time in
+// reverse block order, from the memory-side cache where it still holds it).
+// One block per row over scalar loads, three passes, took (MI355X) 143 us at
+// 64 x 151936, 63 at 4 rows, 536 at 800; the chunks take 22, 11.5 and 285.
+constexpr int kSplitBS = 256, kSplitVPT = 8;
+constexpr int kSplitMax = kWave;  // chunks per row: one per lane in the merge
+
+struct SplitChunk {
+  const float* x;
+  float* row;  // Out's row
+  int64_t beg;
+  int n;
+};
+__device__ __forceinline__ SplitChunk split_chunk(const float* X, float* Out, int64_t dim, int C, int64_t per,
+                                                  int64_t blk) {
+  const int64_t r = blk / C, c = blk % C, beg = c * per;
+  return {X + r * dim + beg, Out + r * dim, beg, int(min(per, dim - beg))};
+}
+__device__ __forceinline__ float load_chunk(const SplitChunk& k, float4 (&v)[kSplitVPT]) {
+  const int n4 = k.n >> 2, ti = 4 * n4 + int(threadIdx.x);
+#pragma unroll
+  for (int j = 0; j < kSplitVPT; ++j) {
+    const int c = int(threadIdx.x) + j * kSplitBS;
+    v[j] = c < n4 ? ld4u(k.x + 4 * c) : make_float4(-INFINITY, -INFINITY, -INFINITY, -INFINITY);
+  }
+  return ti < k.n ? k.x[ti] : -INFINITY;
+}
+
+__global__ __launch_bounds__(kSplitBS) void softmax_split_stats_kernel(const float* __restrict__ X, float* Out,
+                                                                       int64_t dim, int C, int64_t per) {
+  EZ_PROF_WAVE(kProfSoftmax);
+  __shared__ float red[kSplitBS / kWave];
+  const SplitChunk k = split_chunk(X, Out, dim, C, per, blockIdx.x);
+  float4 v[kSplitVPT];
+  const float vt = load_chunk(k, v);
+  float mx = vt;
+#pragma unroll
+  for (int j = 0; j < kSplitVPT; ++j) mx = fmaxf(mx, fmaxf(fmaxf(v[j].x, v[j].y), fmaxf(v[j].z, v[j].w)));
+  mx = block_reduce<kSplitBS / kWave, true>(mx, red);
+  // A chunk of -inf or of the type's lowest value alone (a mask) sums to zero
+  // against the others; a NaN in it still makes the sum NaN.
+  constexpr float kLowest = -3.402823466e38f;
+  const float mb = mx == -INFINITY ? mx : fmaxf(mx * kLog2e, kLowest), ms = mx == -INFINITY ? 0.f : mb;
+  float sum = exp2f(fmaf(vt, kLog2e, -ms));
+#pragma unroll
+  for (int j = 0; j < kSplitVPT; ++j)
+    sum += (exp2f(fmaf(v[j].x, kLog2e, -ms)) + exp2f(fmaf(v[j].y, kLog2e, -ms))) +
+           (exp2f(fmaf(v[j].z, kLog2e, -ms)) + exp2f(fmaf(v[j].w, kLog2e, -ms)));
+  sum = block_reduce<kSplitBS / kWave, false>(sum, red);
+  const int c = int(blockIdx.x % unsigned(C));
+  if (int(threadIdx.x) < C) {
+    float* o = k.row + int64_t(threadIdx.x) * per + 2 * c;
+    o[0] = mb;
+    o[1] = sum;
   }
 }
 
-__global__ __launch_bounds__(1024) void softmax_loop_kernel(const float* __restrict__ X,
-                                                            float* __restrict__ Out, int64_t dim) {
+__global__ __launch_bounds__(kSplitBS) void softmax_split_write_kernel(const float* __restrict__ X, float* Out,
+                                                                       int64_t dim, int C, int64_t per) {
+  EZ_PROF_WAVE(kProfSoftmax);
+  const SplitChunk k = split_chunk(X, Out, dim, C, per, int64_t(gridDim.x) - 1 - blockIdx.x);
+  float* o = k.row + k.beg;
+  const int lane = threadIdx.x & (kWave - 1);
+  const float m = lane < C ? o[2 * lane] : -INFINITY, s = lane < C ? o[2 * lane + 1] : 0.f;
+  float4 v[kSplitVPT];
+  float vt = load_chunk(k, v);
+  const float mb = wave_max(m);
+  const float sum = wave_sum(lane < C ? s * exp2f(m - mb) : 0.f);
+  __syncthreads();  // every wave has read the pairs before the chunk is overwritten
+  const float inv = 1.0f / sum;
+  const int n4 = k.n >> 2, ti = 4 * n4 + int(threadIdx.x);
+#pragma unroll
+  for (int j = 0; j < kSplitVPT; ++j) {
+    const int c = int(threadIdx.x) + j * kSplitBS;
+    if (c < n4)
+      st4u(o + 4 * c, make_float4(exp2f(fmaf(v[j].x, kLog2e, -mb)) * inv, exp2f(fmaf(v[j].y, kLog2e, -mb)) * inv,
+                                  exp2f(fmaf(v[j].z, kLog2e, -mb)) * inv, exp2f(fmaf(v[j].w, kLog2e, -mb)) * inv));
+  }
+  if (ti < k.n) o[ti] = exp2f(fmaf(vt, kLog2e, -mb)) * inv;
+}
+
+// Any other long row (Out overlapping X, or more chunks than the merge
+// holds): one block, three passes.
+__global__ __launch_bounds__(1024) void softmax_loop_kernel(const float* X, float* Out, int64_t dim) {
   EZ_PROF_WAVE(kProfSoftmax);
   __shared__ float red[16];
   const float* x = X + int64_t(blockIdx.x) * dim;
@@ -363,8 +476,7 @@ extern "C" int ezops_rmsnorm_f32(const float* X, float* Out, int64_t rows, int64
                                  hipStream_t s) {
   EZ_REQUIRE(X && Out, "rmsnorm_f32: null pointer");
   EZ_REQUIRE(rows >= 1 && dim >= 1 && rows < (int64_t(1) << 31), "rmsnorm_f32: bad shape");
-  const bool vec = dim % 4 == 0 && aligned16(X) && aligned16(Out);
-  if (!vec || dim > 32768) {
+  if (dim > 32768) {
     hipLaunchKernelGGL(rmsnorm_f32_loop_kernel, dim3(unsigned(rows)), dim3(256), 0, s, X, Out, dim, eps);
   } else if (dim <= 2048) {
     launch_rms_f32<64>(X, Out, rows, dim, eps, s);
@@ -383,8 +495,7 @@ extern "C" int ezops_rmsnorm_bf16(const void* Xv, const void* Wv, void* Ov, int6
   auto O = static_cast<uint16_t*>(Ov);
   EZ_REQUIRE(X && O, "rmsnorm_bf16: null pointer");
   EZ_REQUIRE(rows >= 1 && dim >= 1 && rows < (int64_t(1) << 31), "rmsnorm_bf16: bad shape");
-  const bool vec = dim % 8 == 0 && aligned16(X) && aligned16(O) && (!W || aligned16(W));
-  if (!vec || dim > 65536) {
+  if (dim > 65536) {
     hipLaunchKernelGGL(rmsnorm_bf16_loop_kernel, dim3(unsigned(rows)), dim3(256), 0, s, X, W, O, dim, eps);
   } else if (dim <= 1024) {
     launch_rms_bf16<64>(X, W, O, rows, dim, eps, s);
@@ -411,9 +522,18 @@ int launch_rmsnorm_bf16_packed(const uint16_t* X, const uint16_t* W, uint16_t* O
 extern "C" int ezops_softmax_f32(const float* X, float* Out, int64_t rows, int64_t dim, hipStream_t s) {
   EZ_REQUIRE(X && Out, "softmax_f32: null pointer");
   EZ_REQUIRE(rows >= 1 && dim >= 1 && rows < (int64_t(1) << 31), "softmax_f32: bad shape");
-  const bool vec = dim % 4 == 0 && aligned16(X) && aligned16(Out);
-  if (!vec || dim > 32768) {
-    hipLaunchKernelGGL(softmax_loop_kernel, dim3(unsigned(rows)), dim3(1024), 0, s, X, Out, dim);
+  if (dim > 32768) {
+    // The split launches keep their pairs in Out, so Out must not overlap X.
+    const int64_t C = (dim + 4 * kSplitBS * kSplitVPT - 1) / (4 * kSplitBS * kSplitVPT);
+    const int64_t per = ((dim + C - 1) / C + 3) & ~int64_t(3);
+    const bool apart = X + rows * dim <= Out || Out + rows * dim <= X;
+    if (apart && C <= kSplitMax && rows * C < (int64_t(1) << 31)) {
+      const dim3 g{unsigned(rows * C)}, b{unsigned(kSplitBS)};
+      hipLaunchKernelGGL(softmax_split_stats_kernel, g, b, 0, s, X, Out, dim, int(C), per);
+      hipLaunchKernelGGL(softmax_split_write_kernel, g, b, 0, s, X, Out, dim, int(C), per);
+    } else {
+      hipLaunchKernelGGL(softmax_loop_kernel, dim3(unsigned(rows)), dim3(1024), 0, s, X, Out, dim);
+    }
   } else if (dim <= 2048) {
     launch_softmax<64>(X, Out, rows, dim, s);
   } else if (dim <= 8192) {
