@@ -20,17 +20,18 @@ __device__ __forceinline__ float bf2f(uint16_t h) { return __uint_as_float(uint3
 __device__ __forceinline__ float bf_lo(uint32_t w) { return __uint_as_float(w << 16); }
 __device__ __forceinline__ float bf_hi(uint32_t w) { return __uint_as_float(w & 0xffff0000u); }
 
-// fp32 -> bf16, round to nearest even; NaN stays a quiet NaN.
-__device__ __forceinline__ uint16_t f2bf(float f) {
-  uint32_t u = __float_as_uint(f);
-  if ((u & 0x7fffffffu) > 0x7f800000u) return uint16_t((u >> 16) | 0x40u);
-  u += 0x7fffu + ((u >> 16) & 1u);
-  return uint16_t(u >> 16);
+// fp32 -> bf16, round to nearest even, by the hardware convert
+// (v_cvt_pk_bf16_f32); NaN stays a quiet NaN.  One instruction for two values,
+// where the integer form took about eight each: the RMSNorm prologue of the
+// M = 4 GEMVs is bound by it.
+typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+typedef float f32x2_t __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint32_t cvt_bf2(float lo, float hi) {
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2_t){lo, hi}, bf16x2_t));
 }
+__device__ __forceinline__ uint16_t f2bf(float f) { return __builtin_bit_cast(uint16_t, static_cast<__bf16>(f)); }
 __device__ __forceinline__ float round_bf(float f) { return bf2f(f2bf(f)); }
-__device__ __forceinline__ uint32_t pack_bf2(float lo, float hi) {
-  return uint32_t(f2bf(lo)) | (uint32_t(f2bf(hi)) << 16);
-}
+__device__ __forceinline__ uint32_t pack_bf2(float lo, float hi) { return cvt_bf2(lo, hi); }
 
 // Unpack 8 bf16 held in a uint4 into fp32.
 __device__ __forceinline__ void unpack8(const uint4& v, float (&f)[8]) {
@@ -116,13 +117,6 @@ __device__ __forceinline__ float colgroup_max(float v) {
   v = fmaxf(__uint_as_float(p[0]), __uint_as_float(p[1]));
   const auto q = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
   return fmaxf(__uint_as_float(q[0]), __uint_as_float(q[1]));
-}
-
-typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-typedef float f32x2_t __attribute__((ext_vector_type(2)));
-// Two fp32 -> packed bf16 in one hardware convert (round to nearest even).
-__device__ __forceinline__ uint32_t cvt_bf2(float lo, float hi) {
-  return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2_t){lo, hi}, bf16x2_t));
 }
 
 // s_waitcnt with vmcnt = N and the other counters unconstrained (gfx9 encoding).

@@ -16,6 +16,8 @@
 // registers, then the reference's bf16 staging of the normalised input;
 // M > 4: one staging pass into the workspace) and the residual / SwiGLU
 // epilogues of the decode layer.
+#include <type_traits>
+
 #include "common.h"
 #include "internal.h"
 #include "prof.h"
@@ -730,6 +732,28 @@ __global__ __launch_bounds__(4 * kWave) void linear_xs_kernel(LinearArgs a) {
   }
 }
 
+// c + a . b over 8 bf16 pairs with fp32 accumulation.  DOT2: two products per
+// instruction straight from the packed pairs (v_dot2_f32_bf16): from two batch
+// rows on the kernel is bound by its arithmetic (gate/up at batch 4 46.8 -> 41.5
+// us, down 25.7 -> 23.2).  Otherwise unpacked FMAs, which a single batch row
+// hides under its loads.
+template <bool DOT2>
+__device__ __forceinline__ float dot8(const uint4& a, const uint4& b, float c) {
+  if constexpr (DOT2) {
+    const uint32_t aw[4] = {a.x, a.y, a.z, a.w}, bw[4] = {b.x, b.y, b.z, b.w};
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      c = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, aw[q]), __builtin_bit_cast(bf16x2_t, bw[q]), c, false);
+  } else {
+    float x[8], y[8];
+    unpack8(a, x);
+    unpack8(b, y);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) c = fmaf(x[e], y[e], c);
+  }
+  return c;
+}
+
 // ---------------------------------------------------------------------------
 // Row-block GEMV, M <= 4 and K % 8 == 0, K <= 16384.  A block of 256
 // threads is split into 256 / TPR row groups of TPR threads; each group owns
@@ -811,12 +835,7 @@ __global__ __launch_bounds__(kBlock) void gemv_rows_kernel(LinearArgs a) {
     for (int m = 0; m < M; ++m) {
       ss[m] = 0.f;
 #pragma unroll
-      for (int j = 0; j < CH; ++j) {
-        float x[8];
-        unpack8(xv[m][j], x);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) ss[m] = fmaf(x[e], x[e], ss[m]);
-      }
+      for (int j = 0; j < CH; ++j) ss[m] = dot8<(M > 1)>(xv[m][j], xv[m][j], ss[m]);
       const float v = wave_reduce_uniform<false>(ss[m]);
       if (lane == 0) sred[wave][m] = v;
     }
@@ -846,17 +865,9 @@ __global__ __launch_bounds__(kBlock) void gemv_rows_kernel(LinearArgs a) {
 #pragma unroll
   for (int j = 0; j < CH; ++j) {
 #pragma unroll
-    for (int m = 0; m < M; ++m) {
-      float x[8];
-      unpack8(xv[m][j], x);
+    for (int m = 0; m < M; ++m)
 #pragma unroll
-      for (int r = 0; r < NR; ++r) {
-        float w[8];
-        unpack8(wv[r][j], w);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) acc[m][r] = fmaf(w[e], x[e], acc[m][r]);
-      }
-    }
+      for (int r = 0; r < NR; ++r) acc[m][r] = dot8<(M > 1)>(wv[r][j], xv[m][j], acc[m][r]);
   }
 
 #pragma unroll
@@ -921,33 +932,51 @@ void launch_valu(const LinearArgs& a, hipStream_t s) {
   hipLaunchKernelGGL((gemv_valu_kernel<M, R, U, NORM, SILU>), dim3(blocks), dim3(kGemvBlock), 0, s, a);
 }
 
-// Rows per row group of the row-block GEMV, by chunks per thread (measured
-// on the Qwen3-8B stages: K = 4096 four rows, the QKV projection ran
-// 10.5 / 11.1 / 12.0 us with 4 / 2 / 1; K = 12288 two rows, the down
-// projection 17.8 / 18.4 us with 2 / 1; SwiGLU halves them: two gate and
+// Rows per row group of the row-block GEMV, by chunks per thread.
+//
+// One batch row (measured on the Qwen3-8B stages: K = 4096 four rows, the QKV
+// projection ran 10.5 / 11.1 / 12.0 us with 4 / 2 / 1; K = 12288 two rows, the
+// down projection 17.8 / 18.4 us with 2 / 1; SwiGLU halves them: two gate and
 // two up rows, 32.6 us against 34.5 with one each).  More rows lose at the
 // layer level (config L, batch 1, three alternating runs each: 83.4-85.8 us
 // per layer; four gate + four up rows 86.4-87.1; four down rows alone
 // 86.4-86.7; with eight QKV rows as well 87.6-87.8).
-constexpr int rows_per_group(int ch, bool silu) { return silu ? (ch <= 2 ? 2 : 1) : (ch <= 2 ? 4 : 2); }
+//
+// Two to four batch rows: each block loads (and with the RMSNorm prologue
+// normalises) every row of X, so twice the weight rows halve that work (batch
+// 4, us: Qwen3-8B gate/up 41.5 -> 37.6, o_proj 12.6 -> 9.1, down 23.2 -> 21.5;
+// VL-2B QKV 13.9 -> 8.3), as far as the row chunks fit the registers.
+constexpr int rows_per_group(int m, bool norm, int ch, bool silu) {
+  const int base = silu ? (ch <= 2 ? 2 : 1) : (ch <= 2 ? 4 : 2);
+  const int two = norm ? 2 * base : (silu ? base : 4);
+  return m > 1 && ((silu ? 2 : 1) * two + m) * ch <= 48 ? two : base;
+}
 
 template <int M, int CH, int TPR, bool NORM, bool SILU, bool TAIL>
 void launch_rows_t(const LinearArgs& a, hipStream_t s) {
-  constexpr int RB = rows_per_group(CH, SILU);
+  constexpr int RB = rows_per_group(M, NORM, CH, SILU);
   constexpr int RG = kBlock / TPR;
-  // Small matrices (<= 1024 blocks of RB rows): a quarter of the rows per
-  // group, so four times the blocks share the ramp (GEMV 4096 x 4096, RB 4 /
-  // 2 / 1: 8.0 / 7.7 / 7.5 us; two rows at K = 6144 and 2048 rows, 1024 or
-  // 2048 blocks: 6.20 / 6.24 us).
-  if constexpr (RB == 4) {
-    if ((a.N + RB * RG - 1) / (RB * RG) <= 1024) {
-      const int64_t blocks = (a.N + RG - 1) / RG;
-      hipLaunchKernelGGL((gemv_rows_kernel<M, 1, CH, TPR, NORM, SILU, TAIL>), dim3(unsigned(blocks)), dim3(kBlock), 0, s, a);
-      return;
-    }
-  }
+  auto launch = [&](auto rb) {
+    constexpr int R = decltype(rb)::value;
+    const int64_t blocks = (a.N + R * RG - 1) / (R * RG);
+    hipLaunchKernelGGL((gemv_rows_kernel<M, R, CH, TPR, NORM, SILU, TAIL>), dim3(unsigned(blocks)), dim3(kBlock), 0, s, a);
+  };
   const int64_t blocks = (a.N + RB * RG - 1) / (RB * RG);
-  hipLaunchKernelGGL((gemv_rows_kernel<M, RB, CH, TPR, NORM, SILU, TAIL>), dim3(unsigned(blocks)), dim3(kBlock), 0, s, a);
+  // Small matrices take fewer rows per group, so that more blocks share the
+  // ramp: one batch row, <= 1024 blocks of four rows: one row (GEMV 4096 x 4096,
+  // 4 / 2 / 1 rows: 8.0 / 7.7 / 7.5 us; two rows at K = 6144 and 2048 rows, 1024
+  // or 2048 blocks: 6.20 / 6.24 us).  Two to four: below 1024 blocks of four
+  // rows one row (K <= 4096) or two (4096 x 4096 at batch 4, 4 / 2 / 1 rows: 9.1 /
+  // 10.0 / 12.8 us; 2048 x 2048: 5.1 / 4.7 / 4.7); with the prologue, below 512
+  // blocks half the rows (Qwen3-0.6B QKV at batch 4, 8 / 4 / 1: 6.4 / 5.9 / 8.3).
+  if constexpr (M > 1 && NORM) {
+    if (blocks < 512 && RB > 1) return launch(std::integral_constant<int, (RB > 1 ? RB / 2 : 1)>{});
+  } else if constexpr (M > 1 && !SILU && RB == 4) {
+    if (blocks < 1024) return launch(std::integral_constant<int, (CH <= 2 ? 1 : 2)>{});
+  } else if constexpr (M == 1 && RB == 4) {
+    if (blocks <= 1024) return launch(std::integral_constant<int, 1>{});
+  }
+  launch(std::integral_constant<int, RB>{});
 }
 
 template <int M, int CH, int TPR, bool NORM, bool SILU>
