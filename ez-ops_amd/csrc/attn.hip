@@ -240,7 +240,7 @@ __device__ __forceinline__ int64_t out_index(const AttnArgs& a, int64_t hq, int 
 // index) and the long sequences never start last.  One wave, B <= 64: lane j
 // ranks sequence j against all others, the lane holding rank r is found by
 // ballot.
-__device__ __forceinline__ int rank_to_seq(const int32_t* lens, int B, int r, int lane) {
+__device__ __forceinline__ int rank_to_seq(const int32_t* lens, int B, int r, int lane, int32_t* len) {
   const int32_t Lj = lane < B ? lens[lane] : -1;
   int rank = 0;
   for (int j = 0; j < B; ++j) {
@@ -248,7 +248,21 @@ __device__ __forceinline__ int rank_to_seq(const int32_t* lens, int B, int r, in
     rank += (Lo > Lj) || (Lo == Lj && j < lane);
   }
   const uint64_t hit = __ballot(lane < B && rank == r);
-  return hit ? __ffsll(static_cast<unsigned long long>(hit)) - 1 : r;
+  const int b = hit ? __ffsll(static_cast<unsigned long long>(hit)) - 1 : r;
+  *len = __builtin_amdgcn_readlane(Lj, b);
+  return b;
+}
+
+// Inclusive prefix sum over the 64 lanes (DPP row shifts, then the rows' totals
+// broadcast to the rows behind them).
+__device__ __forceinline__ int wave_scan(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);  // row_shr 1, 2, 4, 8
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // lane 15 of rows 0, 2 to rows 1, 3
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // lane 31 to rows 2, 3
+  return v;
 }
 
 // LAYER: q (and the decoded token's k, v) come from the bf16 QKV projection
@@ -278,31 +292,35 @@ __global__ __launch_bounds__(W * kWave) void attn_split_kernel(AttnArgs a, int n
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // uniform: scalar tile loop
   const int li = lane & 15, lg = lane >> 4;
   int split, kvh, b, nsb = nsplit;  // nsb: splits of this block's sequence
+  // The sequence's length where a ragged batch's block order needed it already
+  // (then the first tile and the cos / sin rows are requested for it, not for
+  // the host's bound).
+  int32_t Lk = 0;
+  bool known = false;
   if (a.split_chunk > 0) {
     // Ragged batch (B <= 64), splits in proportion to the lengths: sequence
-    // j gets ns_j = ceil(len_j / split_chunk) splits per kv head; blocks run
-    // longest sequence first, (kv head, split) within; blocks past the
-    // active ones leave before loading anything.  Lane j < B holds
-    // sequence j's length, rank and first block.
+    // j gets ns_j = ceil(len_j / split_chunk) splits per kv head, blocks in
+    // (sequence, kv head, split) order; blocks past the active ones leave
+    // before loading anything.  Lane j < B holds sequence j's length, and a
+    // wave scan its first block.  (Ordering the sequences longest first cost
+    // ~1000 instructions per block before its first load and balanced nothing:
+    // a block's share is between half a chunk and a chunk whatever its length.
+    // Qwen3-8B layer, 64 ragged sequences up to 4096 rows, paged: attention 122.6
+    // -> 97 us; 16 up to 16384: 85.5 -> 81.)
     const int B = int(a.B);
     int32_t Lj = lane < B ? a.kv_lens[lane] : 0;
     Lj = Lj < 0 ? 0 : (int64_t(Lj) > a.Lh ? int32_t(a.Lh) : Lj);
-    int rank = 0;
-    for (int m = 0; m < B; ++m) {
-      const int32_t Lo = __builtin_amdgcn_readlane(Lj, m);
-      rank += (Lo > Lj) || (Lo == Lj && m < lane);
-    }
-    int ns = int((int64_t(Lj) + a.split_chunk - 1) / a.split_chunk);
+    int ns = int((uint32_t(Lj) + uint32_t(a.split_chunk) - 1) / uint32_t(a.split_chunk));
     ns = ns < 1 ? 1 : (ns > nsplit ? nsplit : ns);
-    int start = 0;
-    for (int m = 0; m < B; ++m)
-      start += __builtin_amdgcn_readlane(rank, m) < rank ? __builtin_amdgcn_readlane(ns, m) * int(a.Hkv) : 0;
+    const int own = lane < B ? ns * int(a.Hkv) : 0, end = wave_scan(own), start = end - own;
     const int blk = int(blockIdx.x);
-    const uint64_t hit = __ballot(lane < B && blk >= start && blk < start + ns * int(a.Hkv));
+    const uint64_t hit = __ballot(lane < B && blk >= start && blk < end);
     if (!hit) return;  // beyond the active blocks (uniform over the block)
     b = __ffsll(static_cast<unsigned long long>(hit)) - 1;
     nsb = __builtin_amdgcn_readlane(ns, b);
     const int off = blk - __builtin_amdgcn_readlane(start, b);
+    Lk = __builtin_amdgcn_readlane(Lj, b);
+    known = true;
     kvh = off / nsb;
     split = off % nsb;
   } else {
@@ -310,8 +328,13 @@ __global__ __launch_bounds__(W * kWave) void attn_split_kernel(AttnArgs a, int n
     const int unit = int(blockIdx.x / unsigned(nsplit));
     kvh = unit % int(a.Hkv);
     b = unit / int(a.Hkv);
-    if (a.sort_lens) b = rank_to_seq(a.kv_lens, int(a.B), b, lane);
+    if (a.sort_lens) {
+      b = rank_to_seq(a.kv_lens, int(a.B), b, lane, &Lk);
+      known = true;
+    }
   }
+  Lk = Lk < 0 ? 0 : (int64_t(Lk) > a.Lh ? int32_t(a.Lh) : Lk);
+  const int64_t Lb = known ? (Lk > 0 ? Lk : 1) : a.Lh;  // bound of the rows requested before the length
   // The length is requested first, ahead of this wave's tile loads, and
   // unconditionally (a dummy address without kv_lens), so that nothing waits
   // for it before its first use.  It is a vector load (an opaque per-lane
@@ -341,7 +364,7 @@ __global__ __launch_bounds__(W * kWave) void attn_split_kernel(AttnArgs a, int n
   // s tps + w, then every W-th, below t_end) -- every block then carries the
   // same bytes, which sets the time when there is one block per CU.
   const int64_t stride = (a.tps > 0 ? int64_t(1) : int64_t(nsb)) * W * kTile;  // distance between a wave's tiles
-  const int64_t t_end = a.tps > 0 ? min(a.Lh, (int64_t(split) + 1) * a.tps * kTile) : a.Lh;
+  const int64_t t_end = a.tps > 0 ? min(Lb, (int64_t(split) + 1) * a.tps * kTile) : Lb;
   uint16_t* slab = &Vs[wave][0];
 
   int64_t t0 = (a.tps > 0 ? int64_t(split) * a.tps + wave : int64_t(split) * W + wave) * kTile;
@@ -369,11 +392,11 @@ __global__ __launch_bounds__(W * kWave) void attn_split_kernel(AttnArgs a, int n
     const uint16_t* vrow = row + (a.H + a.Hkv) * D + int64_t(kvh) * D;
     vv1 = vrow[lane & (D / 2 - 1)];
     vv2 = vrow[(lane & (D / 2 - 1)) + D / 2];
-    // The rows of the host's bound Lh - 1, which is the token position
-    // whenever the sequence is the longest (B = 1 with an exact bound): no
-    // wait for the length before the tile loads go out.  Another position
-    // reloads them once the length is in (below).
-    const int64_t pos_s = a.Lh > 0 ? a.Lh - 1 : 0;
+    // The rows of the known length, or of the host's bound Lh - 1, which is the
+    // token position whenever the sequence is the longest (B = 1 with an exact
+    // bound): no wait for the length before the tile loads go out.  Another
+    // position reloads them once the length is in (below).
+    const int64_t pos_s = Lb - 1;
     rin = load_rope<D>(a.cos ? a.cos + pos_s * D : row, a.sin ? a.sin + pos_s * D : row, lane);
   }
   __builtin_amdgcn_sched_barrier(0);
@@ -387,7 +410,7 @@ __global__ __launch_bounds__(W * kWave) void attn_split_kernel(AttnArgs a, int n
 
   int32_t Lraw;  // read here, behind the tile loads (asm: not hoisted to the load)
   asm volatile("v_readfirstlane_b32 %0, %1" : "=s"(Lraw) : "v"(Lv));
-  int64_t L = a.kv_lens ? int64_t(Lraw) : a.S;
+  int64_t L = known ? int64_t(Lk) : a.kv_lens ? int64_t(Lraw) : a.S;
   L = L < 0 ? 0 : (L > a.Lh ? a.Lh : L);
   // Cache rows read here: [0, Lc) (the layer's decoded token is the virtual row).
   const int64_t Lc = LAYER ? (L > 0 ? L - 1 : 0) : L;
@@ -401,7 +424,7 @@ __global__ __launch_bounds__(W * kWave) void attn_split_kernel(AttnArgs a, int n
     const int64_t pos = L - 1;
     if (L > 0) {
       const bool rope = a.cos != nullptr;
-      if (rope && pos != (a.Lh > 0 ? a.Lh - 1 : 0)) rin = load_rope_sync<D>(a.cos + pos * D, a.sin + pos * D, lane);
+      if (rope && pos != Lb - 1) rin = load_rope_sync<D>(a.cos + pos * D, a.sin + pos * D, lane);
 #pragma unroll
       for (int j = 0; j < NQ; ++j)
         if (wave + j * W < G) finish_head<D>(qin[j], rin, a.qw != nullptr, rope, a.eps, &Qs[wave + j * W][0], lane);
@@ -674,9 +697,18 @@ SplitPlan plan_splits(int64_t B, int64_t Hkv, int64_t Lh, int64_t G, bool balanc
   // 8-wave blocks for few units; groups 8 and 16 keep 4 waves (its accumulators need
   // the register budget of one wave per SIMD).
   const int waves = (units * 4 <= cus && G <= 4) ? 8 : 4;
-  const int64_t target = waves == 8 ? 2 * cus : 8 * cus;  // blocks in flight (4-wave: B=16 layer 211/205/205/212/220 us at 4/6/8/12/16 per CU)
+  const int64_t target = waves == 8 ? 2 * cus : 8 * cus;  // blocks (4-wave: B=16 layer 211/205/205/212/220 us at 4/6/8/12/16 per CU)
   int64_t ns = (target + units - 1) / units;
   const int64_t max_ns = (Lh + int64_t(waves) * kTile - 1) / (int64_t(waves) * kTile);
+  if (waves == 4 && balance) {
+    // Beyond one block for each of the two places on a CU, a split keeps at
+    // least 512 rows: four tiles per wave to carry the block's prologue and
+    // merge.  (Qwen3-8B layer's attention, 64 sequences of 512 rows: one split
+    // 27.8 us, four and a merge launch 63.4 + 4.9; 32 ragged sequences up to 1024
+    // rows 18.9 against 38.0; at least 256 rows: 27.1 + 4.8 and 22.0.)
+    const int64_t fill = (2 * cus + units - 1) / units, rows = Lh / 512;
+    if (ns > fill && ns > rows) ns = fill > rows ? fill : rows;
+  }
   if (ns > max_ns) ns = max_ns;
   if (ns > kMaxSplits) ns = kMaxSplits;
   if (ns < 1) ns = 1;
