@@ -105,42 +105,70 @@ def lib() -> C.CDLL:
     return _lib
 
 
+_fns: dict = {}  # entry points by name, of the library in `_fns_of`
+_fns_of = None
+
+
+def _fn(name: str):
+    """The bound entry point (the library in use can be swapped: ezops.profiling)."""
+    global _fns, _fns_of
+    l = _lib if _lib is not None else lib()
+    if l is not _fns_of:
+        _fns, _fns_of = {}, l
+    fns = _fns
+    fn = fns.get(name)
+    if fn is None:
+        fn = getattr(l, name)
+        fns[name] = fn
+    return fn
+
+
 def call(name: str, *args) -> None:
     """Invoke an int-returning entry point; non-zero status raises RuntimeError."""
-    rc = getattr(lib(), name)(*args)
+    rc = _fn(name)(*args)
     if rc != 0:
         msg = lib().ezops_hip_last_error().decode(errors="replace")
         raise RuntimeError(f"{name} failed ({rc}): {msg}")
 
 
 def size(name: str, *args) -> int:
-    return int(getattr(lib(), name)(*args))
+    return int(_fn(name)(*args))
 
 
 def ptr(t: torch.Tensor | None) -> int | None:
     return None if t is None else t.data_ptr()
 
 
+# The stream handle alone: torch.cuda.current_stream builds a Stream object,
+# about a microsecond of each call.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def stream(device: torch.device | None = None) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    if device is None or device.index is None or _raw_stream is None:
+        return torch.cuda.current_stream(device).cuda_stream
+    return _raw_stream(device.index)
 
 
 def require_gpu(*tensors: torch.Tensor) -> torch.device:
     """All tensors on one GPU; the HIP backend has no CPU path."""
-    dev = None
+    dev = index = None
     for t in tensors:
         if t is None:
             continue
-        if t.device.type != "cuda":
+        if not t.is_cuda:
             raise RuntimeError(f"HIP backend needs GPU tensors, got a tensor on {t.device}")
         if dev is None:
             dev = t.device
-        elif t.device != dev:
+            index = dev.index
+        elif t.get_device() != index:
             raise RuntimeError(f"tensors on different devices: {dev} and {t.device}")
     return dev
 
 
 def check(t: torch.Tensor, name: str, shape: tuple, dtype: torch.dtype) -> None:
+    if t.shape == shape and t.dtype is dtype and t.is_contiguous():
+        return
     if tuple(t.shape) != tuple(shape):
         raise ValueError(f"{name}: expected shape {tuple(shape)}, got {tuple(t.shape)}")
     if t.dtype != dtype:

@@ -27,6 +27,7 @@ class AttnDecodeHipKernel(BaseKernel):
             raise ValueError("batch and seq_len must be >= 1")
         self.B, self.H, self.S, self.D, self.Hkv = batch, num_heads, seq_len, head_dim, num_kv_heads
         self._ws = _hip.Workspace()
+        self._ws_bytes = 0  # by the library, at the first call
 
     def __call__(self, Q: torch.Tensor, K: torch.Tensor, V: torch.Tensor, kv_lens: torch.Tensor | None = None,
                  max_kv_len: int = 0):
@@ -44,8 +45,9 @@ class AttnDecodeHipKernel(BaseKernel):
         if kv_lens is not None:
             _hip.check(kv_lens, "kv_lens", (self.B,), torch.int32)
         Out = torch.empty(self.B, self.H, 1, self.D, dtype=bf, device=dev)
-        nbytes = _hip.size("ezops_attn_decode_workspace_size", self.B, self.H, self.Hkv, self.S, self.D)
-        ws = self._ws.get(nbytes, dev)
+        if not self._ws_bytes:
+            self._ws_bytes = _hip.size("ezops_attn_decode_workspace_size", self.B, self.H, self.Hkv, self.S, self.D)
+        ws = self._ws.get(self._ws_bytes, dev)
         _hip.call("ezops_attn_decode_bf16", Q.data_ptr(), K.data_ptr(), V.data_ptr(), Out.data_ptr(),
                   self.B, self.H, self.Hkv, self.S, self.D, _hip.ptr(kv_lens), int(max_kv_len), 0.0, ws.data_ptr(), ws.numel(),
                   _hip.stream(dev))

@@ -27,6 +27,7 @@ class PagedAttnDecodeHipKernel(BaseKernel):
         self.B, self.H, self.Hkv, self.D = batch, num_heads, num_kv_heads, head_dim
         self.P, self.M, self.NP = page_size, max_pages, num_pages
         self._ws = _hip.Workspace()
+        self._ws_bytes = 0  # by the library, at the first call
 
     def __call__(self, Q: torch.Tensor, K_pages: torch.Tensor, V_pages: torch.Tensor, block_table: torch.Tensor,
                  kv_lens: torch.Tensor, max_kv_len: int = 0):
@@ -40,8 +41,9 @@ class PagedAttnDecodeHipKernel(BaseKernel):
         _hip.check(block_table, "block_table", (self.B, self.M), torch.int32)
         _hip.check(kv_lens, "kv_lens", (self.B,), torch.int32)
         Out = torch.empty(self.B, self.H, 1, self.D, dtype=bf, device=dev)
-        S = self.M * self.P
-        ws = self._ws.get(_hip.size("ezops_attn_decode_workspace_size", self.B, self.H, self.Hkv, S, self.D), dev)
+        if not self._ws_bytes:
+            self._ws_bytes = _hip.size("ezops_attn_decode_workspace_size", self.B, self.H, self.Hkv, self.M * self.P, self.D)
+        ws = self._ws.get(self._ws_bytes, dev)
         _hip.call("ezops_paged_attn_decode_bf16", Q.data_ptr(), K_pages.data_ptr(), V_pages.data_ptr(),
                   Out.data_ptr(), block_table.data_ptr(), kv_lens.data_ptr(), self.B, self.H, self.Hkv, self.D,
                   self.NP, self.P, self.M, int(max_kv_len), 0.0, ws.data_ptr(), ws.numel(), _hip.stream(dev))

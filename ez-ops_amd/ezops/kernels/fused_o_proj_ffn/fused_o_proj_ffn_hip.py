@@ -23,6 +23,7 @@ class FusedOProjFfnHipKernel(BaseKernel):
                     attention_width=num_heads * head_dim)
         self.B, self.HS, self.IS, self.QR = batch, hidden_size, intermediate_size, num_heads * head_dim
         self._ws = _hip.Workspace()
+        self._ws_bytes = 0  # by the library, at the first call
 
     def __call__(self, attn, residual, Wo, post_norm_w, Wg, Wu, Wd):
         dev = _hip.require_gpu(attn, residual, Wo, post_norm_w, Wg, Wu, Wd)
@@ -36,7 +37,9 @@ class FusedOProjFfnHipKernel(BaseKernel):
         _hip.check(Wu, "Wu", (IS, HS), bf)
         _hip.check(Wd, "Wd", (HS, IS), bf)
         out = torch.empty(B, HS, dtype=bf, device=dev)
-        ws = self._ws.get(_hip.size("ezops_o_proj_ffn_workspace_size", B, HS, IS, QR), dev)
+        if not self._ws_bytes:
+            self._ws_bytes = _hip.size("ezops_o_proj_ffn_workspace_size", B, HS, IS, QR)
+        ws = self._ws.get(self._ws_bytes, dev)
         _hip.call("ezops_o_proj_ffn_bf16", attn.data_ptr(), residual.data_ptr(), Wo.data_ptr(),
                   post_norm_w.data_ptr(), Wg.data_ptr(), Wu.data_ptr(), Wd.data_ptr(), out.data_ptr(),
                   B, HS, IS, QR, RMS_EPS, ws.data_ptr(), ws.numel(), _hip.stream(dev))

@@ -26,6 +26,8 @@ class Qwen3DecodeStepHipKernel(BaseKernel):
             raise ValueError("num_layers must be >= 1 and vocab_size >= 0")
         self.L, self.V = num_layers, vocab_size
         self._ws = _hip.Workspace()
+        self._ws_bytes = 0  # by the library, at the first call
+        self._params = self.layer._params * num_layers
 
     def __call__(self, hidden, layers, cos=None, sin=None, final_norm_w=None, lm_head=None, block_table=None):
         k = self.layer
@@ -45,9 +47,6 @@ class Qwen3DecodeStepHipKernel(BaseKernel):
             raise ValueError("cos/sin given without rope_theta")
         if paged:
             _hip.check(block_table, "block_table", (B, S // k.page_size), torch.int32)
-            kv_shape = (k.num_pages, Hkv, k.page_size, D)
-        else:
-            kv_shape = (B, Hkv, S, D)
         if self.V:
             _hip.check(lm_head, "lm_head", (self.V, HS), bf)
             if final_norm_w is not None:
@@ -55,34 +54,33 @@ class Qwen3DecodeStepHipKernel(BaseKernel):
         nw_n = 4 if k.norm_weights else 0
         out = torch.empty(B, HS, dtype=bf, device=dev)
         logits = torch.empty(B, self.V, dtype=bf, device=dev) if self.V else None
-        lens = k._lens(dev)
-        params = (_hip.Qwen3LayerParams * self.L)()
+        lens = _hip.ptr(k._lens(dev))
+        pcos, psin = _hip.ptr(cos), _hip.ptr(sin)
+        params = (_hip.Qwen3LayerParams * self.L).from_buffer_copy(self._params)
+        check, kv_shape, names = _hip.check, k._kv_shape, k._weights + (k._norms if nw_n else ())
         for i, layer in enumerate(layers):
             if len(layer) != 6 + nw_n:
                 raise ValueError(f"layer {i}: expected {6 + nw_n} tensors, got {len(layer)}")
-            Kc, Vc, Wqkv, Wo, Wgu, Wd = layer[:6]
-            nw = list(layer[6:]) if nw_n else [None] * 4
             _hip.require_gpu(*layer)
-            _hip.check(Kc, f"layer {i} K_cache", kv_shape, bf)
-            _hip.check(Vc, f"layer {i} V_cache", kv_shape, bf)
-            _hip.check(Wqkv, f"layer {i} Wqkv", ((H + 2 * Hkv) * D, HS), bf)
-            _hip.check(Wo, f"layer {i} Wo", (HS, H * D), bf)
-            _hip.check(Wgu, f"layer {i} Wgu", (2 * IS, HS), bf)
-            _hip.check(Wd, f"layer {i} Wd", (HS, IS), bf)
-            for t, n, name in zip(nw, (HS, D, D, HS), ("in_norm_w", "q_norm_w", "k_norm_w", "post_norm_w")):
-                if t is not None:
-                    _hip.check(t, f"layer {i} {name}", (n,), bf)
+            try:
+                check(layer[0], "K_cache", kv_shape, bf)
+                check(layer[1], "V_cache", kv_shape, bf)
+                for t, (name, shape) in zip(layer[2:], names):
+                    if t is not None:
+                        check(t, name, shape, bf)
+            except ValueError as e:
+                raise ValueError(f"layer {i} {e}") from None
             p = params[i]
-            p.B, p.S, p.HS, p.IS, p.H, p.Hkv, p.D, p.eps = B, S, HS, IS, H, Hkv, D, RMS_EPS
-            p.hidden = hidden.data_ptr() if i == 0 else None
-            p.K_cache, p.V_cache = Kc.data_ptr(), Vc.data_ptr()
-            p.Wqkv, p.Wo, p.Wgu, p.Wd = Wqkv.data_ptr(), Wo.data_ptr(), Wgu.data_ptr(), Wd.data_ptr()
-            p.in_norm_w, p.q_norm_w, p.k_norm_w, p.post_norm_w = (_hip.ptr(t) for t in nw)
-            p.cos, p.sin = _hip.ptr(cos), _hip.ptr(sin)
-            p.kv_lens = _hip.ptr(lens)
-            p.max_kv_len = max(k.kv_lens) if k.kv_lens else 0
-            p.out = out.data_ptr() if i == self.L - 1 else None
-        ws = self._ws.get(_hip.size("ezops_qwen3_decode_step_workspace_size", params, self.L, self.V), dev)
+            p.K_cache, p.V_cache = layer[0].data_ptr(), layer[1].data_ptr()
+            p.Wqkv, p.Wo, p.Wgu, p.Wd = (t.data_ptr() for t in layer[2:6])
+            if nw_n:
+                p.in_norm_w, p.q_norm_w, p.k_norm_w, p.post_norm_w = map(_hip.ptr, layer[6:])
+            p.cos, p.sin, p.kv_lens = pcos, psin, lens
+        params[0].hidden = hidden.data_ptr()
+        params[self.L - 1].out = out.data_ptr()
+        if not self._ws_bytes:
+            self._ws_bytes = _hip.size("ezops_qwen3_decode_step_workspace_size", params, self.L, self.V)
+        ws = self._ws.get(self._ws_bytes, dev)
         _hip.call("ezops_qwen3_decode_step_bf16", params, self.L, _hip.ptr(block_table),
                   k.num_pages if paged else 0, k.page_size if paged else 0, _hip.ptr(final_norm_w),
                   _hip.ptr(lm_head), self.V, _hip.ptr(logits), ws.data_ptr(), ws.numel(), _hip.stream(dev))

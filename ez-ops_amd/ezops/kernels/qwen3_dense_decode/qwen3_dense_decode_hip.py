@@ -38,7 +38,15 @@ class Qwen3DenseDecodeHipKernel(BaseKernel):
             num_pages = batch * (seq_len // page_size) if num_pages is None else num_pages
         self.page_size, self.num_pages = page_size, num_pages
         self._ws = _hip.Workspace()
+        self._ws_bytes = 0  # by the library, at the first call
         self._lens_dev: dict = {}
+        # the parameter block's shapes, copied for each call, and the inputs' shapes
+        B, S, HS, IS, H, D, Hkv = batch, seq_len, hidden_size, intermediate_size, num_heads, head_dim, num_kv_heads
+        self._params = bytes(_hip.Qwen3LayerParams(B=B, S=S, HS=HS, IS=IS, H=H, Hkv=Hkv, D=D, eps=RMS_EPS,
+                                                   max_kv_len=max(self.kv_lens) if self.kv_lens else 0))
+        self._kv_shape = (B, Hkv, S, D) if page_size is None else (num_pages, Hkv, page_size, D)
+        self._weights = (("Wqkv", ((H + 2 * Hkv) * D, HS)), ("Wo", (HS, H * D)), ("Wgu", (2 * IS, HS)), ("Wd", (HS, IS)))
+        self._norms = (("in_norm_w", (HS,)), ("q_norm_w", (D,)), ("k_norm_w", (D,)), ("post_norm_w", (HS,)))
 
     def _lens(self, dev):
         if self.kv_lens is None:
@@ -64,38 +72,32 @@ class Qwen3DenseDecodeHipKernel(BaseKernel):
         cos, sin = extra[-2:] if self.rope else (None, None)
         dev = _hip.require_gpu(hidden, K_cache, V_cache, Wqkv, Wo, Wgu, Wd, *extra, *([] if bt is None else [bt]))
         bf = torch.bfloat16
-        B, S, HS, IS, H, D, Hkv = self.B, self.S, self.HS, self.IS, self.H, self.D, self.Hkv
-        _hip.check(hidden, "hidden", (B, HS), bf)
-        if bt is None:
-            kv_shape = (B, Hkv, S, D)
-        else:
-            kv_shape = (self.num_pages, Hkv, self.page_size, D)
-            _hip.check(bt, "block_table", (B, S // self.page_size), torch.int32)
-        _hip.check(K_cache, "K_cache", kv_shape, bf)
-        _hip.check(V_cache, "V_cache", kv_shape, bf)
-        _hip.check(Wqkv, "Wqkv", ((H + 2 * Hkv) * D, HS), bf)
-        _hip.check(Wo, "Wo", (HS, H * D), bf)
-        _hip.check(Wgu, "Wgu", (2 * IS, HS), bf)
-        _hip.check(Wd, "Wd", (HS, IS), bf)
-        for t, n, name in zip(nw, (HS, D, D, HS), ("in_norm_w", "q_norm_w", "k_norm_w", "post_norm_w")):
+        check = _hip.check
+        check(hidden, "hidden", (self.B, self.HS), bf)
+        if bt is not None:
+            check(bt, "block_table", (self.B, self.S // self.page_size), torch.int32)
+        check(K_cache, "K_cache", self._kv_shape, bf)
+        check(V_cache, "V_cache", self._kv_shape, bf)
+        for t, (name, shape) in zip((Wqkv, Wo, Wgu, Wd), self._weights):
+            check(t, name, shape, bf)
+        for t, (name, shape) in zip(nw, self._norms):
             if t is not None:
-                _hip.check(t, name, (n,), bf)
+                check(t, name, shape, bf)
         if self.rope:
-            _hip.check(cos, "cos", (S, D), bf)
-            _hip.check(sin, "sin", (S, D), bf)
-        out = torch.empty(B, HS, dtype=bf, device=dev)
-        lens = self._lens(dev)
-        p = _hip.Qwen3LayerParams(
-            B=B, S=S, HS=HS, IS=IS, H=H, Hkv=Hkv, D=D, eps=RMS_EPS,
-            hidden=hidden.data_ptr(), K_cache=K_cache.data_ptr(), V_cache=V_cache.data_ptr(),
-            Wqkv=Wqkv.data_ptr(), Wo=Wo.data_ptr(), Wgu=Wgu.data_ptr(), Wd=Wd.data_ptr(),
-            in_norm_w=_hip.ptr(nw[0]), q_norm_w=_hip.ptr(nw[1]), k_norm_w=_hip.ptr(nw[2]),
-            post_norm_w=_hip.ptr(nw[3]), cos=_hip.ptr(cos), sin=_hip.ptr(sin), kv_lens=_hip.ptr(lens),
-            max_kv_len=max(self.kv_lens) if self.kv_lens else 0,
-            out=out.data_ptr(),
-        )
+            check(cos, "cos", (self.S, self.D), bf)
+            check(sin, "sin", (self.S, self.D), bf)
+        out = torch.empty(self.B, self.HS, dtype=bf, device=dev)
+        p = _hip.Qwen3LayerParams.from_buffer_copy(self._params)
+        p.hidden, p.K_cache, p.V_cache = hidden.data_ptr(), K_cache.data_ptr(), V_cache.data_ptr()
+        p.Wqkv, p.Wo, p.Wgu, p.Wd = Wqkv.data_ptr(), Wo.data_ptr(), Wgu.data_ptr(), Wd.data_ptr()
+        p.in_norm_w, p.q_norm_w, p.k_norm_w, p.post_norm_w = map(_hip.ptr, nw)
+        p.cos, p.sin = _hip.ptr(cos), _hip.ptr(sin)
+        p.kv_lens = _hip.ptr(self._lens(dev))
+        p.out = out.data_ptr()
         pp = ctypes.byref(p)
-        ws = self._ws.get(_hip.size("ezops_qwen3_layer_workspace_size", pp), dev)
+        if not self._ws_bytes:
+            self._ws_bytes = _hip.size("ezops_qwen3_layer_workspace_size", pp)
+        ws = self._ws.get(self._ws_bytes, dev)
         if bt is None:
             _hip.call("ezops_qwen3_dense_decode_bf16", pp, ws.data_ptr(), ws.numel(), _hip.stream(dev))
         else:

@@ -35,6 +35,7 @@ class Qwen3PrefillHipKernel(BaseKernel):
         self._host = (cu, self.past_lens)
         self._dev: dict = {}
         self._ws = _hip.Workspace()
+        self._ws_bytes = 0  # by the library, at the first call
 
     def _meta(self, dev):
         t = self._dev.get(dev)
@@ -84,7 +85,9 @@ class Qwen3PrefillHipKernel(BaseKernel):
             max_kv_len=0, out=out.data_ptr(),
         )
         pp = ctypes.byref(p)
-        ws = self._ws.get(_hip.size("ezops_qwen3_prefill_workspace_size", pp, T), dev)
+        if not self._ws_bytes:
+            self._ws_bytes = _hip.size("ezops_qwen3_prefill_workspace_size", pp, T)
+        ws = self._ws.get(self._ws_bytes, dev)
         _hip.call("ezops_qwen3_prefill_bf16", pp, T, cu.data_ptr(), max(self.q_lens), _hip.ptr(bt),
                   self.num_pages or 0, self.page_size or 0, ws.data_ptr(), ws.numel(), _hip.stream(dev))
         return out
