@@ -7,7 +7,7 @@
 // neighbouring tiles) against MT 16-row batch blocks: each weight fragment is
 // read from LDS once and meets MT activation fragments.
 //
-//   * NW waves split K into 256-wide chunks; a chunk of a 16-row tile (8 KiB)
+//   * 4 waves split K into 256-wide chunks; a chunk of a 16-row tile (8 KiB)
 //     lands in LDS by DMA (buffer_load_dwordx4 ... lds) in 512-byte row pieces
 //     at XOR-swizzled 16-byte slots (piece c of row r at slot c ^ r), through a
 //     two-stage ring per wave, as in linear_mfma_kernel: no block barriers in
@@ -22,10 +22,11 @@
 //
 // Bound: HBM (weights) up to 32 rows; at 64 the X fragments, MT / T times the
 // weight bytes through each CU's L1.  Measured (MI355X, Qwen3-8B, kernel
-// traces, this kernel against 16 rows per read of W): 64 rows: gate/up 46.5
-// against 131.7 us, QKV 22.6 / 38.1, o_proj + down 61 / 116; the decode layer
-// at 64 rows 400 -> 244 us.  32 rows: gate/up 37.1, QKV 16.4 us (16 rows: 35.7,
-// 15.6).
+// traces, this kernel against 16 rows per read of W): 64 rows: gate/up 45
+// against 131.7 us, QKV 18.7 / 38.1, o_proj + down 49 / 116.  32 rows: gate/up
+// 37.1, QKV 14.1 us (16 rows: 35.7, 15.6).  The X traffic costs about 1 us per
+// 18 MB over the chip; requesting X a whole chunk ahead (two chunks in
+// registers) changed nothing.
 #include "common.h"
 #include "internal.h"
 #include "prof.h"
@@ -36,6 +37,7 @@ namespace ez {
 EZ_PROF_DEFINE(linear_mt)
 namespace {
 
+constexpr int NW = 4;                  // waves per block, splitting K
 constexpr int kKC = 256;               // K elements per chunk
 constexpr int kSteps = kKC / 32;       // MFMA k-steps per chunk
 constexpr int kHalf = kSteps / 2;      // k-steps per X buffer
@@ -101,7 +103,7 @@ __device__ __forceinline__ void store4(const LinearArgs& a, bool vec, int64_t m,
 // XP: X in the packed layout (K % 32 == 0).  Wave operands as in
 // linear_mfma_kernel: lane 16 g + i of the A operand holds W[row + i][8 g ..],
 // of B X[m + i][8 g ..], C[4 g + j][i] in register j.
-template <int T, bool SILU, int MT, int NW, bool XP>
+template <int T, bool SILU, int MT, bool XP>
 __global__ __launch_bounds__(NW * kWave) void linear_mt_kernel(LinearArgs a, bool vec) {
   static_assert(T == 1 || T == 2, "one or two 16-row tiles");
   static_assert(!SILU || T == 2, "SwiGLU: gate and up tile");
@@ -295,24 +297,25 @@ __global__ __launch_bounds__(NW * kWave) void linear_mt_kernel(LinearArgs a, boo
   wait_vm<0>();  // no DMA into this block's LDS outlives it
 }
 
-template <int T, bool SILU, int MT, int NW>
+template <int T, bool SILU, int MT>
 void launch_x(const LinearArgs& a, unsigned gx, bool vec, hipStream_t s) {
   const dim3 grid(gx, unsigned((a.M + 16 * MT - 1) / (16 * MT))), block(NW * kWave);
-  if (a.x_packed) hipLaunchKernelGGL((linear_mt_kernel<T, SILU, MT, NW, true>), grid, block, 0, s, a, vec);
-  else hipLaunchKernelGGL((linear_mt_kernel<T, SILU, MT, NW, false>), grid, block, 0, s, a, vec);
+  if (a.x_packed) hipLaunchKernelGGL((linear_mt_kernel<T, SILU, MT, true>), grid, block, 0, s, a, vec);
+  else hipLaunchKernelGGL((linear_mt_kernel<T, SILU, MT, false>), grid, block, 0, s, a, vec);
 }
 
 template <int MT>
 void launch_m(const LinearArgs& a, bool vec, hipStream_t s) {
   const int64_t cus = num_cus(), tiles = (a.N + 15) / 16;
   auto grid = [&](int64_t t, int64_t slots) { return unsigned(t < slots ? t : slots); };
-  if (a.epi == kEpiSilu) return launch_x<2, true, MT, 4>(a, grid(tiles, cus), vec, s);
-  // Two-tile blocks (each X fragment meets 32 weight rows) where every CU still
-  // has at least two of them (an LM head).
-  if (tiles >= 4 * cus) return launch_x<2, false, MT, 4>(a, grid((a.N + 31) / 32, cus), vec, s);
-  // One tile per CU: 8 waves split K.  More: 4-wave blocks, two to a CU.
-  if (tiles <= cus) return launch_x<1, false, MT, 8>(a, unsigned(tiles), vec, s);
-  launch_x<1, false, MT, 4>(a, grid(tiles, 2 * cus), vec, s);
+  if (a.epi == kEpiSilu) return launch_x<2, true, MT>(a, grid(tiles, cus), vec, s);
+  // Two-tile blocks (each X fragment meets 32 weight rows) where most CUs still
+  // have one: Qwen3-8B QKV (192 blocks) at 64 rows 22.1 -> 18.7 us, at 32 16.1 ->
+  // 14.1; o_proj and down on half the CUs lose (together 49 -> 59 us).
+  if (4 * tiles > 5 * cus) return launch_x<2, false, MT>(a, grid((a.N + 31) / 32, cus), vec, s);
+  // Else 16-row tiles, 4 waves each (8 waves splitting K: VL-2B QKV + o_proj +
+  // down at 40 rows 35.4 against 29.5 us, 0.6B at 64 rows 26.7 against 24.0).
+  launch_x<1, false, MT>(a, grid(tiles, 2 * cus), vec, s);
 }
 
 }  // namespace
