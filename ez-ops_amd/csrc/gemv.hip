@@ -8,9 +8,9 @@
 //     1 KiB of a row and every x chunk serves all rows of the group.
 //   * gemv_valu (M <= 4, longer rows): one wave per R weight rows streaming
 //     16-byte chunks in a loop.
-//   * linear_mt (M > 16, linear_mt.hip): up to 64 batch rows per read of W.
-//   * linear_mfma (4 < M <= 16): v_mfma_f32_16x16x32_bf16 on 16-row weight tiles
-//     against 16 batch rows; the K range is split over the 4 waves of a
+//   * linear_mt (M > 4, linear_mt.hip): up to 64 batch rows per read of W.
+//   * linear_mfma (4 < M <= 16, SwiGLU and the shapes it is unrolled for):
+//     v_mfma_f32_16x16x32_bf16 on 16-row weight tiles against 16 batch rows; the K range is split over the 4 waves of a
 //     block and the partial tiles are summed through LDS.
 // They fuse the RMSNorm prologue (M <= 4: statistics from the x chunks in
 // registers, then the reference's bf16 staging of the normalised input;
@@ -1024,20 +1024,23 @@ void launch_valu_m(const LinearArgs& a, hipStream_t s) {
   }
 }
 
-template <bool SILU, int NW, int TPB = 1>
-void launch_mfma_nw(const LinearArgs& a, hipStream_t s) {
+// 4-wave blocks of 16 weight rows (SwiGLU: 16 gate + 16 up).
+template <bool SILU>
+void launch_mfma_tiles(const LinearArgs& a, hipStream_t s) {
   constexpr int T = SILU ? 2 : 1;
-  const dim3 grid(unsigned((a.N + 15) / 16), unsigned((a.M + 15) / 16)), block(NW * kWave);
+  const dim3 grid(unsigned((a.N + 15) / 16), unsigned((a.M + 15) / 16)), block(4 * kWave);
   const int64_t nchunks = (a.K + kMfmaKC - 1) / kMfmaKC;
-  const int64_t cpw = nchunks % NW == 0 ? nchunks / NW : 0;
-#define EZ_MFMA_LAUNCH(C) hipLaunchKernelGGL((linear_mfma_kernel<T, SILU, C, NW, 1>), grid, block, 0, s, a)
-  switch (cpw) {
-    case 1: EZ_MFMA_LAUNCH(1); break;
-    case 2: EZ_MFMA_LAUNCH(2); break;
-    case 4: EZ_MFMA_LAUNCH(4); break;
-    case 6: EZ_MFMA_LAUNCH(6); break;
-    default: EZ_MFMA_LAUNCH(0); break;
+#define EZ_MFMA_LAUNCH(C) hipLaunchKernelGGL((linear_mfma_kernel<T, SILU, C, 4, 1>), grid, block, 0, s, a)
+  if constexpr (SILU) {
+    switch (nchunks % 4 == 0 ? nchunks / 4 : 0) {
+      case 1: EZ_MFMA_LAUNCH(1); return;
+      case 2: EZ_MFMA_LAUNCH(2); return;
+      case 4: EZ_MFMA_LAUNCH(4); return;
+      case 6: EZ_MFMA_LAUNCH(6); return;
+      default: break;
+    }
   }
+  EZ_MFMA_LAUNCH(0);
 #undef EZ_MFMA_LAUNCH
 }
 
@@ -1063,34 +1066,32 @@ void launch_mfma_stream(const LinearArgs& a, int64_t cus, hipStream_t s) {
   hipLaunchKernelGGL((linear_mfma_kernel<1, false, 4, 4, -1>), grid, block, 0, s, a);
 }
 
-// Blocks of 16 weight rows (T=2: 16 gate + 16 up).  An 8-wave T=1 block
-// holds 136 KB of LDS, one per CU; when the tiles outnumber the CUs but not
-// twice over (QKV at 6144 rows: 384 tiles), 4-wave blocks (68 KB) share a CU
-// two by two so every tile runs in the first round instead of 1.5 rounds.
+// M > 4.  Up to 16 rows SwiGLU and two shapes of the plain stages keep the
+// kernels unrolled for them; everything else runs linear_mt (its own X extents
+// permitting).
 template <bool SILU>
 void launch_mfma(const LinearArgs& a, hipStream_t s) {
+  const int64_t tx = (a.N + 15) / 16, cus = num_cus();
+  const int64_t nchunks = (a.K + kMfmaKC - 1) / kMfmaKC;
+  const bool mt = linear_mt_supported(a);
+  if (a.M > 16 && mt) return launch_linear_mt(a, s);
   if constexpr (SILU) {
     // gate/up of the model shapes (K = 4096: 4 chunks per wave): 3 or 2
     // tiles per CU run as multi-tile blocks, one per CU.
-    const int64_t tx = (a.N + 15) / 16, cus = num_cus();
-    const int64_t nchunks = (a.K + kMfmaKC - 1) / kMfmaKC;
     if (nchunks == 16 && a.K % kMfmaKC == 0 && (tx == 3 * cus || tx == 2 * cus)) {
       const dim3 grid(unsigned(cus), unsigned((a.M + 15) / 16)), block(4 * kWave);
       if (tx == 3 * cus) hipLaunchKernelGGL((linear_mfma_kernel<2, true, 4, 4, 3>), grid, block, 0, s, a);
       else hipLaunchKernelGGL((linear_mfma_kernel<2, true, 4, 4, 2>), grid, block, 0, s, a);
       return;
     }
-    launch_mfma_nw<true, 4>(a, s);
+    launch_mfma_tiles<true>(a, s);
   } else {
-    const int64_t tiles = ((a.N + 15) / 16) * ((a.M + 15) / 16), cus = num_cus();
     // 16 < rows per CU <= 24 (QKV of the model: 6144 rows, 24 per CU): one
     // 24-row block per CU instead of 16-row tiles two to some CUs.
-    const int64_t nchunks = (a.K + kMfmaKC - 1) / kMfmaKC;
     if (a.M <= 16 && a.N > 16 * cus && a.N <= 24 * cus) launch_mfma_r2<8>(a, s);
-    else if ((a.N + 15) / 16 >= 4 * cus && nchunks == 16 && a.K % kMfmaKC == 0)
-      launch_mfma_stream(a, cus, s);
-    else if (tiles > cus && tiles <= 2 * cus) launch_mfma_nw<false, 4>(a, s);
-    else launch_mfma_nw<false, 8>(a, s);
+    else if (tx >= 4 * cus && nchunks == 16 && a.K % kMfmaKC == 0) launch_mfma_stream(a, cus, s);
+    else if (mt) launch_linear_mt(a, s);
+    else launch_mfma_tiles<false>(a, s);
   }
 }
 
@@ -1178,8 +1179,7 @@ int launch_linear(const LinearArgs& a, hipStream_t s) {
       b.ldx = a.K;
       b.norm = 0;
     }
-    if (linear_mt_supported(b)) launch_linear_mt(b, s);
-    else silu ? launch_mfma<true>(b, s) : launch_mfma<false>(b, s);
+    silu ? launch_mfma<true>(b, s) : launch_mfma<false>(b, s);
   }
   return launch_status("linear");
 }

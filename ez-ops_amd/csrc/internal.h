@@ -45,11 +45,11 @@ struct LinearArgs {
 };
 
 int launch_linear(const LinearArgs& a, hipStream_t s);
-// The same for M > 16 without the RMSNorm prologue (linear_mt.hip), operands
+// The same for M > 4 without the RMSNorm prologue (linear_mt.hip), operands
 // already checked by launch_linear; linear_mt_supported: 32-bit extents of a
 // 64-row block of X.
 inline bool linear_mt_supported(const LinearArgs& a) {
-  return a.M > 16 && a.K < (int64_t(1) << 23) && (a.x_packed || a.ldx < (int64_t(1) << 23));
+  return a.M > 4 && a.K < (int64_t(1) << 23) && (a.x_packed || a.ldx < (int64_t(1) << 23));
 }
 void launch_linear_mt(const LinearArgs& a, hipStream_t s);
 

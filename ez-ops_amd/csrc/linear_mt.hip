@@ -1,4 +1,4 @@
-// Skinny linear layers for 17 to 64 batch rows (and more, 64 at a time):
+// Skinny linear layers for 5 to 64 batch rows (and more, 64 at a time):
 // Y[M, N] = epi(X[M, K] . W[N, K]^T), every weight byte read once per 64 rows.
 //
 // The 16-row kernels of gemv.hip read W once per 16 batch rows (grid.y), so at
@@ -26,7 +26,9 @@
 // against 131.7 us, QKV 18.7 / 38.1, o_proj + down 49 / 116.  32 rows: gate/up
 // 37.1, QKV 14.1 us (16 rows: 35.7, 15.6).  The X traffic costs about 1 us per
 // 18 MB over the chip; requesting X a whole chunk ahead (two chunks in
-// registers) changed nothing.
+// registers) changed nothing.  Up to 16 rows: VL-2B QKV + o_proj + down 24.4 ->
+// 21.8 us, 0.6B 18.4 -> 16.7, the 0.6B LM head 110 -> 56 against the 16-row kernel
+// (Qwen3-8B o_proj + down 29.9 / 29.6).
 #include "common.h"
 #include "internal.h"
 #include "prof.h"
@@ -320,11 +322,12 @@ void launch_m(const LinearArgs& a, bool vec, hipStream_t s) {
 
 }  // namespace
 
-// M > 16, operands checked by launch_linear (16-byte rows, 32-bit extents).
+// M > 4, operands checked by launch_linear (16-byte rows, 32-bit extents).
 void launch_linear_mt(const LinearArgs& a, hipStream_t s) {
   const bool vec = a.ldy % 4 == 0 && (reinterpret_cast<uintptr_t>(a.Y) & 7) == 0 &&
                    (a.epi != kEpiResid || (a.ldr % 4 == 0 && (reinterpret_cast<uintptr_t>(a.res) & 7) == 0));
-  if (a.M <= 32) launch_m<2>(a, vec, s);
+  if (a.M <= 16) launch_m<1>(a, vec, s);
+  else if (a.M <= 32) launch_m<2>(a, vec, s);
   else if (a.M <= 48) launch_m<3>(a, vec, s);
   else launch_m<4>(a, vec, s);
 }
