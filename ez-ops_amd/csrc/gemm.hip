@@ -199,10 +199,8 @@ __global__ __launch_bounds__(kGThreads, WPE) void gemm_bf16_kernel(GemmArgs a) {
       if constexpr (RA > 1) frag_issue<kRA>(aa, f[1]);
       frag_issue<0>(ba, f[RA]);
       if (DPS * s < ND) dma1(DPS * s, r0, r1, k0b, dst);
-      if constexpr (RA > 2) {
-        frag_issue<2 * kRA>(aa, f[2]);
-        frag_issue<3 * kRA>(aa, f[3]);
-      }
+      if constexpr (RA > 2) frag_issue<2 * kRA>(aa, f[2]);
+      if constexpr (RA > 3) frag_issue<3 * kRA>(aa, f[3]);
       if constexpr (RB > 1) frag_issue<kRB>(ba, f[RA + 1]);
       if constexpr (RB > 2) frag_issue<2 * kRB>(ba, f[RA + 2]);
       if (DPS > 1 && DPS * s + 1 < ND) dma1(DPS * s + 1, r0, r1, k0b, dst);
@@ -349,17 +347,19 @@ constexpr TileCost kTiles[] = {
     {256, 256, 1, 75.f, 112.f},  // 0
     {256, 192, 1, 57.f, 90.f},   // 1 (not SwiGLU)
     {256, 128, 1, 46.f, 68.f},   // 2
-    {128, 128, 2, 38.f, 69.f},   // 3: two blocks per CU, K-steps of 64
+    {128, 128, 2, 38.f, 75.f},   // 3: two blocks per CU, K-steps of 64
     {128, 128, 1, 29.f, 44.f},   // 4: K-steps of 128
     {64, 128, 1, 23.f, 29.f},    // 5: K-steps of 128 (not SwiGLU)
+    {192, 256, 1, 57.f, 90.f},   // 6
 };
 
 // The shape with the least estimated time: full rounds at `hi`, a part-filled
 // last round between `lo` and `hi`.  Against 256-wide tiles for every GEMM of at
 // least half a round and 256 x 128 below (the rule before), measured in us at
 // Qwen3-8B's (QKV, o_proj, gate/up, down): 700 tokens 61 / 64 / 198 / 187 ->
-// 50 / 35 / 180 / 100; 256 tokens 67 / 70 / 90 / 190 -> 25 / 24 / 80 / 80;
-// 2048 tokens QKV 90 -> 84, o_proj 86 -> 68, down 247 -> 190.
+// 50 / 35 / 152 / 100; 256 tokens 67 / 70 / 90 / 190 -> 25 / 24 / 80 / 80;
+// 2048 tokens QKV 90 -> 84, o_proj 86 -> 68, down 247 -> 186; 3000 tokens QKV
+// 167 -> 142, o_proj 95 -> 87, down 264 -> 246.
 int pick_tile(int64_t M, int64_t N, bool swiglu, int64_t cus) {
   int best = 0;
   float least = 0.f;
@@ -385,6 +385,7 @@ void launch_gemm(const GemmArgs& a, hipStream_t s) {
     case 2: return launch_tile<SWIGLU, 2, 2, 2, 2, 64, 3, 3, 2>(a, s);
     case 3: return launch_tile<SWIGLU, 1, 2, 2, 2, 64, 2, 3, 4>(a, s);
     case 4: return launch_tile<SWIGLU, 1, 2, 2, 2, 128, 2, 3, 2>(a, s);
+    case 6: return launch_tile<SWIGLU, 3, 2, 1, 4, 64, 2, 3, 2>(a, s);
     default: if constexpr (!SWIGLU) return launch_tile<SWIGLU, 1, 1, 1, 4, 128, 3, 3, 2>(a, s);
   }
 }

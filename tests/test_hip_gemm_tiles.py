@@ -31,7 +31,9 @@ def _data(M, N, K, seed=0):
 
 # (M, N) chosen so that, on 256 CUs, each tile shape of the table is picked:
 # 256x256, 256x192, 256x128, 128x128 (two per CU), 128x128 (K-steps of 128), 64x128
-SHAPES = [(4000, 4090), (2040, 6136), (2040, 4090), (1000, 6136), (1020, 4090), (200, 6136), (1, 130), (65, 72)]
+# (three times), 192x256
+SHAPES = [(4000, 4090), (2040, 6136), (2040, 4090), (700, 6136), (1020, 4090), (200, 6136), (1, 130), (65, 72),
+          (3000, 4090)]
 
 
 @pytest.mark.parametrize("M,N", SHAPES)
@@ -50,12 +52,12 @@ def test_gemm_tile_edges(M, N, K, resid):
 def test_gemm_tile_shapes_bit_identical(K):
     X, W = _data(4000, 6136, K, seed=1)
     full = _gemm(X, W)
-    for M, N in [(4000, 4090), (2040, 6136), (2040, 4090), (1000, 6136), (1020, 4090), (200, 6136), (5, 40)]:
+    for M, N in [(4000, 4090), (2040, 6136), (2040, 4090), (700, 6136), (1020, 4090), (200, 6136), (5, 40), (3000, 4090)]:
         assert torch.equal(_gemm(X[:M], W[:N]), full[:M, :N]), (M, N)
 
 
-# gate/up: 256x256, 256x128, 128x128 twice
-@pytest.mark.parametrize("M,IS", [(500, 12288), (4000, 2048), (700, 12288), (120, 12288), (1, 128), (130, 384)])
+# gate/up: 256x256 twice, 128x128 (two per CU), 192x256, 128x128
+@pytest.mark.parametrize("M,IS", [(500, 12288), (740, 12288), (4000, 2048), (600, 12288), (120, 12288), (1, 128), (130, 384)])
 @pytest.mark.parametrize("K", [40, 128, 520])
 def test_gemm_swiglu_tiles_match_plain(M, IS, K):
     X, W = _data(M, 2 * IS, K, seed=2)
