@@ -268,20 +268,34 @@ extern "C" int ezops_qwen3_decode_step_bf16(const ezops_qwen3_layer* layers, int
 // -> o_proj GEMM (+residual) -> RMSNorm -> gate/up GEMM -> SwiGLU -> down
 // GEMM (+residual).
 namespace {
+// Chunks of up to 64 tokens run the decode layer's linear stages, which read W
+// once for up to 64 rows; the GEMM's smallest tile costs its whole K loop however
+// few rows are live.  Layer, us, GEMM with 256-row tiles / with the tile table /
+// linear stages: Qwen3-8B 64 tokens 409 / ~200 / 144, 5 tokens 385 / ~200 / 92; VL-2B
+// 60 tokens 232 / - / 78; 0.6B 154 / - / 58.  At 96 tokens the stages would read W
+// twice (GEMM 205).  HS <= 16384 is the limit of the RMSNorm staging.
+constexpr int64_t kSkinnyTokens = 64;
+bool skinny(const ezops_qwen3_layer* p, int64_t T) { return T <= kSkinnyTokens && p->HS <= 16384; }
+
 struct PrefillBufs {
   uint16_t *xn, *qkv, *att, *h, *gu, *act;
+  char* ffn;  // skinny: run_ffn's workspace
 };
 size_t prefill_ws(const ezops_qwen3_layer* p, int64_t T, PrefillBufs* b, char* base) {
   const int64_t QR = p->H * p->D, QKV = QR + 2 * p->Hkv * p->D;
   Carve c{base};
   auto take = [&](int64_t elems) { return c.take<uint16_t>(size_t(elems) * 2); };
   PrefillBufs t{};
-  t.xn = take(T * p->HS);
+  t.xn = take(packed_rows(T) * p->HS);
   t.qkv = take(T * QKV);
   t.att = take(T * QR);
-  t.h = take(T * p->HS);
-  t.gu = take(T * 2 * p->IS);
-  t.act = take(T * p->IS);
+  if (skinny(p, T)) {
+    t.ffn = c.take<char>(ffn_ws(T, p->HS, p->IS));
+  } else {
+    t.h = take(T * p->HS);
+    t.gu = take(T * 2 * p->IS);
+    t.act = take(T * p->IS);
+  }
   if (b) *b = t;
   return size_t(c.p - base);
 }
@@ -343,6 +357,20 @@ extern "C" int ezops_qwen3_prefill_bf16(const ezops_qwen3_layer* p, int64_t T, c
   int rc = check_qk_norm_rope(r);
   if (!rc) rc = check_prefill_attn(a);
   if (rc) return rc;
+
+  if (skinny(p, T)) {
+    LinearArgs l{};
+    l.X = hidden; l.ldx = HS; l.W = W(p->Wqkv); l.Y = w.qkv; l.ldy = QKV;
+    l.M = T; l.N = QKV; l.K = HS; l.norm = 1; l.norm_w = W(p->in_norm_w);
+    l.eps = p->eps; l.epi = kEpiStore; l.xn_ws = w.xn;
+    rc = launch_linear(l, s);
+    if (!rc) rc = launch_qk_norm_rope(r, s);
+    if (!rc) rc = launch_prefill_attn(a, s);
+    if (!rc)
+      rc = run_ffn(w.att, false, hidden, W(p->Wo), W(p->post_norm_w), W(p->Wgu), W(p->Wgu) + IS * HS, W(p->Wd),
+                   static_cast<uint16_t*>(p->out), T, HS, IS, QR, p->eps, w.ffn, s);
+    return rc;
+  }
 
   rc = ezops_rmsnorm_bf16(hidden, p->in_norm_w, w.xn, T, HS, p->eps, s);
   if (!rc) rc = gemm_bf16(w.xn, HS, W(p->Wqkv), w.qkv, QKV, nullptr, T, QKV, HS, s);
