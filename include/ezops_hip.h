@@ -49,7 +49,7 @@ int ezops_gemv_bf16(const void* A, const void* B, void* C, int64_t N, int64_t K,
 
 /* Skinny bf16 linear layer: Y[m, n] = sum_k X[m, k] * W[n, k] for m < M.
  * X [M, K] (row stride ldx), W [N, K], Y [M, N] (row stride ldy); M >= 1.
- * Rows are processed 16 at a time with MFMA when M > 4.
+ * MFMA when M > 4, W read once per 64 rows.
  * Replaces: the `x @ W.T` projections inside the fused decode kernels
  * (ezops/kernels/fused_o_proj_ffn/fused_o_proj_ffn_triton.py:31-231,
  * ezops/kernels/qwen3_dense_decode/qwen3_dense_decode_triton.py:37-271). */
