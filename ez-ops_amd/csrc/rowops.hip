@@ -156,6 +156,33 @@ __global__ __launch_bounds__(256) void rmsnorm_bf16_loop_kernel(const uint16_t* 
 }
 
 // ------------------------------------------------------------------ softmax
+// exp(x - mx) as exp2((x - a) log2e - b) with a and b of the row's maximum.  Up to
+// |mx| = 256 a = 0 and b = mx log2e: one FMA, whose rounding of b (2^-16 at most) is
+// common to the row and cancels.  That rounding grows with mx -- up to 64 at 1e9, and
+// beyond exp2's range at 1e10 -- and b overflows from 2.4e38 on, so larger maxima (a
+// row of the type's lowest value alone: a full mask) are subtracted first, a = mx:
+// exact for x within a factor of two of mx, and any other x is at least 128 below it
+// and weighs nothing.
+struct ExpBase {
+  float a, b;
+};
+__device__ __forceinline__ ExpBase exp_base(float mx) {
+  return fabsf(mx) < 256.f ? ExpBase{0.f, mx * kLog2e} : ExpBase{mx, 0.f};
+}
+__device__ __forceinline__ float exp_rel(float x, const ExpBase& e) { return exp2f(fmaf(x - e.a, kLog2e, -e.b)); }
+// The same for values in registers: subtracts a where it is not zero (uniform over
+// the row: no instruction per element otherwise, which cost up to 4%) and returns b.
+template <int VPT>
+__device__ __forceinline__ float shift_row(float mx, float4 (&v)[VPT], float& vt) {
+  const ExpBase e = exp_base(mx);
+  if (e.a != 0.f) {
+#pragma unroll
+    for (int j = 0; j < VPT; ++j) v[j] = make_float4(v[j].x - e.a, v[j].y - e.a, v[j].z - e.a, v[j].w - e.a);
+    vt -= e.a;
+  }
+  return e.b;
+}
+
 // A block per row, the row in registers (dim <= 4 * BS * VPT): one read, one
 // write.  The last dim % 4 elements sit in the first threads.
 template <int BS, int VPT>
@@ -177,7 +204,7 @@ __global__ __launch_bounds__(BS) void softmax_reg_kernel(const float* __restrict
 #pragma unroll
   for (int j = 0; j < VPT; ++j) mx = fmaxf(mx, fmaxf(fmaxf(v[j].x, v[j].y), fmaxf(v[j].z, v[j].w)));
   mx = block_reduce<BS / kWave, true>(fmaxf(mx, vt), red);
-  const float mb = mx * kLog2e;
+  const float mb = shift_row(mx, v, vt);
   vt = exp2f(fmaf(vt, kLog2e, -mb));
   float sum = vt;
 #pragma unroll
@@ -200,8 +227,8 @@ __global__ __launch_bounds__(BS) void softmax_reg_kernel(const float* __restrict
 
 // Rows too long for one block's registers, cut into C chunks of `per` floats
 // (<= 4 kSplitBS kSplitVPT; 2 C <= every chunk) over two launches, so that a
-// few long rows fill the chip.  The first writes each chunk's (maximum in
-// log2 units, sum of exponentials) to every chunk's place in Out -- chunk k
+// few long rows fill the chip.  The first writes each chunk's (maximum, sum of
+// exponentials relative to it) to every chunk's place in Out -- chunk k
 // holds the row's C pairs in its first 2 C floats -- and the second reads its
 // chunk's copy, merges the pairs and overwrites the chunk.  Each block of the
 // second touches its own chunk alone, so no block waits for another; the
@@ -239,25 +266,23 @@ __global__ __launch_bounds__(kSplitBS) void softmax_split_stats_kernel(const flo
   __shared__ float red[kSplitBS / kWave];
   const SplitChunk k = split_chunk(X, Out, dim, C, per, blockIdx.x);
   float4 v[kSplitVPT];
-  const float vt = load_chunk(k, v);
+  float vt = load_chunk(k, v);
   float mx = vt;
 #pragma unroll
   for (int j = 0; j < kSplitVPT; ++j) mx = fmaxf(mx, fmaxf(fmaxf(v[j].x, v[j].y), fmaxf(v[j].z, v[j].w)));
   mx = block_reduce<kSplitBS / kWave, true>(mx, red);
-  // A chunk of -inf or of the type's lowest value alone (a mask) sums to zero
-  // against the others; a NaN in it still makes the sum NaN.
-  constexpr float kLowest = -3.402823466e38f;
-  const float mb = mx == -INFINITY ? mx : fmaxf(mx * kLog2e, kLowest), ms = mx == -INFINITY ? 0.f : mb;
-  float sum = exp2f(fmaf(vt, kLog2e, -ms));
+  // A chunk of -inf alone (a mask) sums to zero; a NaN in it still makes the sum NaN.
+  const float mb = mx == -INFINITY ? 0.f : shift_row(mx, v, vt);
+  float sum = exp2f(fmaf(vt, kLog2e, -mb));
 #pragma unroll
   for (int j = 0; j < kSplitVPT; ++j)
-    sum += (exp2f(fmaf(v[j].x, kLog2e, -ms)) + exp2f(fmaf(v[j].y, kLog2e, -ms))) +
-           (exp2f(fmaf(v[j].z, kLog2e, -ms)) + exp2f(fmaf(v[j].w, kLog2e, -ms)));
+    sum += (exp2f(fmaf(v[j].x, kLog2e, -mb)) + exp2f(fmaf(v[j].y, kLog2e, -mb))) +
+           (exp2f(fmaf(v[j].z, kLog2e, -mb)) + exp2f(fmaf(v[j].w, kLog2e, -mb)));
   sum = block_reduce<kSplitBS / kWave, false>(sum, red);
   const int c = int(blockIdx.x % unsigned(C));
   if (int(threadIdx.x) < C) {
     float* o = k.row + int64_t(threadIdx.x) * per + 2 * c;
-    o[0] = mb;
+    o[0] = mx;
     o[1] = sum;
   }
 }
@@ -271,9 +296,12 @@ __global__ __launch_bounds__(kSplitBS) void softmax_split_write_kernel(const flo
   const float m = lane < C ? o[2 * lane] : -INFINITY, s = lane < C ? o[2 * lane + 1] : 0.f;
   float4 v[kSplitVPT];
   float vt = load_chunk(k, v);
-  const float mb = wave_max(m);
-  const float sum = wave_sum(lane < C ? s * exp2f(m - mb) : 0.f);
+  // A chunk's sum is relative to its own base: exp(base - the row's base) as exp_rel.
+  const float mx = wave_max(m);
+  const ExpBase e = exp_base(mx), ec = exp_base(m);
+  const float sum = wave_sum(lane < C ? s * exp2f(fmaf(ec.a - e.a, kLog2e, ec.b - e.b)) : 0.f);
   __syncthreads();  // every wave has read the pairs before the chunk is overwritten
+  const float mb = shift_row(mx, v, vt);
   const float inv = 1.0f / sum;
   const int n4 = k.n >> 2, ti = 4 * n4 + int(threadIdx.x);
 #pragma unroll
@@ -296,12 +324,12 @@ __global__ __launch_bounds__(1024) void softmax_loop_kernel(const float* X, floa
   float mx = -INFINITY;
   for (int64_t i = threadIdx.x; i < dim; i += 1024) mx = fmaxf(mx, x[i]);
   mx = block_reduce<16, true>(mx, red);
-  const float mb = mx * kLog2e;
+  const ExpBase e = exp_base(mx);
   float sum = 0.f;
-  for (int64_t i = threadIdx.x; i < dim; i += 1024) sum += exp2f(fmaf(x[i], kLog2e, -mb));
+  for (int64_t i = threadIdx.x; i < dim; i += 1024) sum += exp_rel(x[i], e);
   sum = block_reduce<16, false>(sum, red);
   const float inv = 1.0f / sum;
-  for (int64_t i = threadIdx.x; i < dim; i += 1024) o[i] = exp2f(fmaf(x[i], kLog2e, -mb)) * inv;
+  for (int64_t i = threadIdx.x; i < dim; i += 1024) o[i] = exp_rel(x[i], e) * inv;
 }
 
 // --------------------------------------------------------------- full sum

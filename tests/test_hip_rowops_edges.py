@@ -56,12 +56,34 @@ def test_softmax_chunked_nonfinite():
     _softmax(X, Out)
     want = torch.softmax(X.double().cpu(), -1)
     got = Out.double().cpu()
-    torch.testing.assert_close(got[[0, 5]], want[[0, 5]], rtol=1e-5, atol=1e-6)
+    torch.testing.assert_close(got[[0, 4, 5]], want[[0, 4, 5]], rtol=1e-5, atol=1e-6)
     assert torch.isnan(got[1:4]).all()
-    short = X[4:5, :1000].contiguous()
-    one = torch.empty_like(short)
-    _softmax(short, one)
-    assert torch.isfinite(got[4]).all() == torch.isfinite(one).all()  # the lowest value: as the one-block kernel
+
+
+# one block per row of 64 / 256 / 1024 threads, rows in chunks, and in place (the three-pass kernel beyond 32768)
+@pytest.mark.parametrize("dim", [1000, 5001, 20000, 40003])
+@pytest.mark.parametrize("inplace", [False, True])
+def test_softmax_large_maxima(dim, inplace):
+    """Finite rows far from zero, where exp(x - max) must come from the difference: a full mask of the type's lowest
+    value, of -1e10 or of the largest value, values near +-256 (where the formula changes) and near +-3e38, and a
+    maximum on either side of 256 in one chunk alone.  Bar: the op's (rtol 1e-5, atol 1e-6) of torch's fp64 softmax."""
+    big = torch.finfo(torch.float32).max
+    base = torch.randn(10, dim, generator=torch.Generator().manual_seed(dim)) * 3
+    X = base.clone()
+    X[0], X[1], X[2] = -big, -1e10, big
+    X[3] = base[3] - 1e6
+    X[4] = base[4] + 250.0  # maxima about 260
+    X[5] = base[5] - 262.0
+    X[6, : dim // 2], X[6, dim // 2:] = 3e38, -3e38
+    X[7, dim // 3:] = -big
+    X[8, dim - 1], X[8, 0] = 300.0, 296.0
+    X[9] = base[9] - 300.0
+    X[9, 1] = 5.0
+    want = torch.softmax(X.double(), -1)
+    X = X.to(DEV)
+    Out = X if inplace else torch.empty_like(X)
+    _softmax(X, Out)
+    torch.testing.assert_close(Out.double().cpu(), want, rtol=1e-5, atol=1e-6)
 
 
 @pytest.mark.parametrize("dim", [1, 7, 513, 1025, 2050, 8197, 16391, 32767, 65535])
