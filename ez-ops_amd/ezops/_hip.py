@@ -105,17 +105,19 @@ def lib() -> C.CDLL:
     return _lib
 
 
-_fns: dict = {}  # entry points by name, of the library in `_fns_of`
-_fns_of = None
+_entries: tuple = (None, {})  # (library, its entry points by name): read and replaced as one
 
 
 def _fn(name: str):
-    """The bound entry point (the library in use can be swapped: ezops.profiling)."""
-    global _fns, _fns_of
-    l = _lib if _lib is not None else lib()
-    if l is not _fns_of:
-        _fns, _fns_of = {}, l
-    fns = _fns
+    """The bound entry point (the library in use can be swapped, also by another thread: ezops.profiling)."""
+    global _entries
+    l = _lib
+    if l is None:
+        l = lib()
+    of, fns = _entries
+    if of is not l:
+        fns = {}
+        _entries = (l, fns)
     fn = fns.get(name)
     if fn is None:
         fn = getattr(l, name)
