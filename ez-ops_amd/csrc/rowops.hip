@@ -336,7 +336,6 @@ __global__ __launch_bounds__(1024) void softmax_loop_kernel(const float* X, floa
 // Stage 1: block b sums a fixed, strided share of the float4s into
 // partial[b]; the last block to finish sums partial[0..G) in index order.
 // The grid size depends only on n, so the result is bitwise reproducible.
-typedef float f32x4v_t __attribute__((ext_vector_type(4)));
 constexpr int kSumBlock = 256;
 constexpr int kSumUnroll = 8;
 constexpr int kSumMaxBlocks = 1024;  // 512: 1e8 67.5 against 65.7 us, 2^28 177 against 163
@@ -352,8 +351,7 @@ int64_t sum_blocks(int64_t n) {
 
 template <bool NT>
 __global__ __launch_bounds__(kSumBlock) void sum_kernel(const float* __restrict__ A, int64_t n,
-                                                        bool vec, float* __restrict__ partial,
-                                                        int* counter, float* __restrict__ Out) {
+                                                        float* __restrict__ partial, int* counter, float* __restrict__ Out) {
   EZ_PROF_WAVE(kProfSum);
   __shared__ float red[kSumBlock / kWave];
   const int64_t G = gridDim.x;
@@ -361,38 +359,43 @@ __global__ __launch_bounds__(kSumBlock) void sum_kernel(const float* __restrict_
   float acc[kSumUnroll];
 #pragma unroll
   for (int u = 0; u < kSumUnroll; ++u) acc[u] = 0.f;
-  int64_t tail_start = 0;
-  if (vec) {
-    // The last, partial batch goes out at once like the full ones, clamped, the
-    // values past the end dropped (one load at a time it was up to seven round
-    // trips).
-    auto ld = [](const f32x4v_t* p) { return NT ? __builtin_nontemporal_load(p) : *p; };
-    const f32x4v_t* a4 = reinterpret_cast<const f32x4v_t*>(A);
-    const int64_t n4 = n >> 2;
-    int64_t i = int64_t(blockIdx.x) * kSumBlock + threadIdx.x;
-    for (; i + (kSumUnroll - 1) * stride < n4; i += kSumUnroll * stride) {
-      f32x4v_t v[kSumUnroll];
+  // 16-byte loads at any element address (see ld4u).  (An array that starts off 16
+  // bytes went one float at a time: n = 1e6 15.7 -> 4.9 us, 1e7 37 -> 11.8, 1e8 179 ->
+  // 68; aligned it is 4.9, 11.4 and 65.)  The last, partial batch
+  // goes out at once like the full ones, clamped, the values past the end dropped
+  // (one load at a time it was up to seven round trips).
+  auto ld = [](const f32x4u_t* p) { return NT ? __builtin_nontemporal_load(p) : *p; };
+  const f32x4u_t* a4 = reinterpret_cast<const f32x4u_t*>(A);
+  const int64_t n4 = n >> 2;
+  int64_t i = int64_t(blockIdx.x) * kSumBlock + threadIdx.x;
+  // Loads in flight: the whole batch, but two of the streamed arrays, whose eight
+  // would lie in as many DRAM pages (8 against 2: n = 1e8 78 against 65 us, 2^28 197
+  // against 157; below the caches' size 8 against 2: 1e5 4.2 / 5.0, 1e7 11.4 / 12.9).
+  constexpr int F = NT ? 2 : kSumUnroll;
+  for (; i + (kSumUnroll - 1) * stride < n4; i += kSumUnroll * stride) {
 #pragma unroll
-      for (int u = 0; u < kSumUnroll; ++u) v[u] = ld(a4 + i + u * stride);
+    for (int q = 0; q < kSumUnroll; q += F) {
+      f32x4u_t v[F];
 #pragma unroll
-      for (int u = 0; u < kSumUnroll; ++u) acc[u] += (v[u].x + v[u].y) + (v[u].z + v[u].w);
+      for (int u = 0; u < F; ++u) v[u] = ld(a4 + i + (q + u) * stride);
+#pragma unroll
+      for (int u = 0; u < F; ++u) acc[q + u] += (v[u].x + v[u].y) + (v[u].z + v[u].w);
+      if (NT) __builtin_amdgcn_sched_barrier(0);
     }
-    if (i < n4) {
-      f32x4v_t v[kSumUnroll];
-#pragma unroll
-      for (int u = 0; u < kSumUnroll; ++u) {
-        const int64_t j = i + u * stride;
-        v[u] = ld(a4 + (j < n4 ? j : n4 - 1));
-      }
-#pragma unroll
-      for (int u = 0; u < kSumUnroll; ++u)
-        acc[u] += i + u * stride < n4 ? (v[u].x + v[u].y) + (v[u].z + v[u].w) : 0.f;
-    }
-    tail_start = n4 << 2;
   }
-  // scalar remainder (all of it when A is not 16-byte aligned)
-  for (int64_t i = tail_start + int64_t(blockIdx.x) * kSumBlock + threadIdx.x; i < n; i += stride)
-    acc[1] += A[i];
+  if (i < n4) {
+    f32x4u_t v[kSumUnroll];
+#pragma unroll
+    for (int u = 0; u < kSumUnroll; ++u) {
+      const int64_t j = i + u * stride;
+      v[u] = ld(a4 + (j < n4 ? j : n4 - 1));
+    }
+#pragma unroll
+    for (int u = 0; u < kSumUnroll; ++u)
+      acc[u] += i + u * stride < n4 ? (v[u].x + v[u].y) + (v[u].z + v[u].w) : 0.f;
+  }
+  // the last n % 4 elements
+  if (const int64_t t = 4 * n4 + threadIdx.x; blockIdx.x == 0 && t < n) acc[1] += A[t];
   float s = 0.f;
 #pragma unroll
   for (int u = 0; u < kSumUnroll; ++u) s += acc[u];
@@ -412,6 +415,7 @@ __global__ __launch_bounds__(kSumBlock) void sum_kernel(const float* __restrict_
 //                    locality, ~20% faster than grid-striding on MI355X),
 //                    8 float4 per thread per trip, non-temporal stores.
 constexpr int kProbeUnroll = 8;
+typedef float f32x4v_t __attribute__((ext_vector_type(4)));
 
 // Grid-stride read.  NT = 0 allocates in the caches (the cache flush of the
 // benchmarks); NT = 1 streams with the non-temporal hint on a 32-blocks-per-CU
@@ -607,9 +611,9 @@ extern "C" int ezops_reduce_sum_f32(const float* A, float* Out, int64_t n, void*
   // would read data from HBM that a previous pass left in the caches (n = 1e6
   // 7.5 -> 11.4).
   if (n >= (int64_t(1) << 25))
-    hipLaunchKernelGGL(sum_kernel<true>, dim3(unsigned(G)), dim3(kSumBlock), 0, s, A, n, aligned16(A), partial, counter, Out);
+    hipLaunchKernelGGL(sum_kernel<true>, dim3(unsigned(G)), dim3(kSumBlock), 0, s, A, n, partial, counter, Out);
   else
-    hipLaunchKernelGGL(sum_kernel<false>, dim3(unsigned(G)), dim3(kSumBlock), 0, s, A, n, aligned16(A), partial, counter, Out);
+    hipLaunchKernelGGL(sum_kernel<false>, dim3(unsigned(G)), dim3(kSumBlock), 0, s, A, n, partial, counter, Out);
   return launch_status("reduce_sum_f32");
 }
 

@@ -107,3 +107,25 @@ def test_rmsnorm_any_row(dim, dtype, off):
     torch.cuda.synchronize()
     torch.testing.assert_close(Out.double().cpu(), want, **tol)
     assert (buf[off + rows * dim:] == 5.0).all() and (buf[:off] == 5.0).all()
+
+
+# batches of 256 threads x 8 float4, the block counts' bounds, partial batches, the streamed arrays
+@pytest.mark.parametrize("n", [1, 3, 4, 1023, 8191, 8193, 32771, 1000003, 4194307, (1 << 25) - 3, (1 << 25) + 8197,
+                               (3 << 24) - 1, (3 << 24) + 8197])
+def test_sum_any_alignment(n):
+    """Full sum of an array that starts at any element: the same bits as at 16 bytes, within 1e-6 of fp64 (fp32 partial
+    sums of non-negative terms: chains of at most 64 values, then a tree), and nothing outside [0, n) in it."""
+    A = torch.rand(n, generator=torch.Generator(device=DEV).manual_seed(n), device=DEV)
+    buf = torch.full((n + 32,), float("nan"), device=DEV)
+    ws = torch.zeros(max(256, _hip.size("ezops_reduce_sum_workspace_size", n)), dtype=torch.uint8, device=DEV)
+    got = []
+    for off in (16, 17, 18, 19):
+        buf.fill_(float("nan"))
+        buf[off:off + n] = A
+        Out = torch.zeros(1, device=DEV)
+        _hip.call("ezops_reduce_sum_f32", buf.data_ptr() + 4 * off, Out.data_ptr(), n, ws.data_ptr(), ws.numel(),
+                  _hip.stream())
+        got.append(float(Out))
+    want = float(A.double().sum())
+    assert abs(got[0] - want) <= 1e-6 * want
+    assert got[1:] == got[:1] * 3
