@@ -169,3 +169,15 @@ def test_batched_linear_rejects_huge_k():
     d, K = 4096, 1 << 26
     rc = lib.ezops_linear_bf16(d, K, d, d, 16, 8, 16, K, None)
     assert rc == _hip.EINVAL and b"2^26" in lib.ezops_hip_last_error()
+
+
+def test_sum_blocks_by_length():
+    """The sum's partials, one per block: a block per 8192 values up to 128 blocks, per 32768 from 2^22 on, at most 1024;
+    never fewer for a longer array (a workspace serves every shorter one)."""
+    blocks = lambda n: (_hip.lib().ezops_reduce_sum_workspace_size(n) - 256) // 4  # noqa: E731  (rounded up to 64)
+    up = lambda g: -(-g // 64) * 64  # noqa: E731
+    for n, g in ((1, 1), (8192, 1), (8193, 2), (600000, 74), (1 << 20, 128), ((1 << 20) + 1, 128), (1 << 22, 128),
+                 ((1 << 22) + 1, 129), (10**7, 306), (1 << 25, 1024), (1 << 28, 1024)):
+        assert blocks(n) == up(g), n
+    sizes = [blocks(n) for n in range(1, 1 << 23, 4099)]
+    assert sizes == sorted(sizes)

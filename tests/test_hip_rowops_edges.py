@@ -110,7 +110,7 @@ def test_rmsnorm_any_row(dim, dtype, off):
 
 
 # batches of 256 threads x 8 float4, the block counts' bounds, partial batches, the streamed arrays
-@pytest.mark.parametrize("n", [1, 3, 4, 1023, 8191, 8193, 32771, 1000003, 4194307, (1 << 25) - 3, (1 << 25) + 8197,
+@pytest.mark.parametrize("n", [1, 3, 4, 1023, 8191, 8193, 32771, 1000003, (1 << 20) + 1, 4194307, (1 << 25) - 3, (1 << 25) + 8197,
                                (3 << 24) - 1, (3 << 24) + 8197])
 def test_sum_any_alignment(n):
     """Full sum of an array that starts at any element: the same bits as at 16 bytes, within 1e-6 of fp64 (fp32 partial
