@@ -609,11 +609,12 @@ extern "C" int ezops_reduce_sum_f32(const float* A, float* Out, int64_t n, void*
   const int64_t G = sum_blocks(n);
   int* counter = static_cast<int*>(ws);
   float* partial = reinterpret_cast<float*>(static_cast<char*>(ws) + 256);
-  // Arrays of at least half the memory-side cache (256 MB) are streamed with the
-  // non-temporal hint: n = 1e8 69.3 -> 64.9 us, 2^28 179 -> 163; below, the hint
-  // would read data from HBM that a previous pass left in the caches (n = 1e6
-  // 7.5 -> 11.4).
-  if (n >= (int64_t(1) << 25))
+  // Arrays of at least three quarters of the memory-side cache (256 MB) are streamed
+  // with the non-temporal hint; below, the hint would read from HBM what a previous
+  // pass left in the caches (n = 1e6 7.5 -> 11.4 us).  A repeated pass / a pass over
+  // other data, us, without and with it: 3.4e7 29.4 / 30.8 and 31.0 / 32.0, 5e7 37.6 /
+  // 39.1 and 39.2 / 39.8, 6.7e7 48.7 / 51.8 and 47.9 / 48.4, 1e8 70 / 69 and 65 / 65.
+  if (n >= (int64_t(3) << 24))
     hipLaunchKernelGGL(sum_kernel<true>, dim3(unsigned(G)), dim3(kSumBlock), 0, s, A, n, partial, counter, Out);
   else
     hipLaunchKernelGGL(sum_kernel<false>, dim3(unsigned(G)), dim3(kSumBlock), 0, s, A, n, partial, counter, Out);
