@@ -9,8 +9,9 @@
 //   * gemv_valu (M <= 4, longer rows): one wave per R weight rows streaming
 //     16-byte chunks in a loop.
 //   * linear_mt (M > 4, linear_mt.hip): up to 64 batch rows per read of W.
-//   * linear_mfma (4 < M <= 16, SwiGLU and the shapes it is unrolled for):
-//     v_mfma_f32_16x16x32_bf16 on 16-row weight tiles against 16 batch rows; the K range is split over the 4 waves of a
+//   * linear_mfma (4 < M <= 16: SwiGLU and the shapes it is unrolled for; above
+//     that narrow matrices): v_mfma_f32_16x16x32_bf16 on 16-row weight tiles
+//     against 16 batch rows; the K range is split over the 4 or 8 waves of a
 //     block and the partial tiles are summed through LDS.
 // They fuse the RMSNorm prologue (M <= 4: statistics from the x chunks in
 // registers, then the reference's bf16 staging of the normalised input;
@@ -1070,23 +1071,20 @@ void launch_valu_m(const LinearArgs& a, hipStream_t s) {
   }
 }
 
-// 4-wave blocks of 16 weight rows (SwiGLU: 16 gate + 16 up).
-template <bool SILU>
-void launch_mfma_tiles(const LinearArgs& a, hipStream_t s) {
+// Blocks of 16 weight rows (SwiGLU: 16 gate + 16 up) by 16 batch rows, NW waves.
+template <bool SILU, int NW>
+void launch_mfma_nw(const LinearArgs& a, hipStream_t s) {
   constexpr int T = SILU ? 2 : 1;
-  const dim3 grid(unsigned((a.N + 15) / 16), unsigned((a.M + 15) / 16)), block(4 * kWave);
+  const dim3 grid(unsigned((a.N + 15) / 16), unsigned((a.M + 15) / 16)), block(NW * kWave);
   const int64_t nchunks = (a.K + kMfmaKC - 1) / kMfmaKC;
-#define EZ_MFMA_LAUNCH(C) hipLaunchKernelGGL((linear_mfma_kernel<T, SILU, C, 4, 1>), grid, block, 0, s, a)
-  if constexpr (SILU) {
-    switch (nchunks % 4 == 0 ? nchunks / 4 : 0) {
-      case 1: EZ_MFMA_LAUNCH(1); return;
-      case 2: EZ_MFMA_LAUNCH(2); return;
-      case 4: EZ_MFMA_LAUNCH(4); return;
-      case 6: EZ_MFMA_LAUNCH(6); return;
-      default: break;
-    }
+#define EZ_MFMA_LAUNCH(C) hipLaunchKernelGGL((linear_mfma_kernel<T, SILU, C, NW, 1>), grid, block, 0, s, a)
+  switch (nchunks % NW == 0 ? nchunks / NW : 0) {
+    case 1: EZ_MFMA_LAUNCH(1); break;
+    case 2: EZ_MFMA_LAUNCH(2); break;
+    case 4: EZ_MFMA_LAUNCH(4); break;
+    case 6: EZ_MFMA_LAUNCH(6); break;
+    default: EZ_MFMA_LAUNCH(0); break;
   }
-  EZ_MFMA_LAUNCH(0);
 #undef EZ_MFMA_LAUNCH
 }
 
@@ -1112,15 +1110,34 @@ void launch_mfma_stream(const LinearArgs& a, int64_t cus, hipStream_t s) {
   hipLaunchKernelGGL((linear_mfma_kernel<1, false, 4, 4, -1>), grid, block, 0, s, a);
 }
 
-// M > 4.  Up to 16 rows SwiGLU and two shapes of the plain stages keep the
-// kernels unrolled for them; everything else runs linear_mt (its own X extents
-// permitting).
+// Above 16 batch rows, few weight rows: a block per 16 weight rows and 16 batch rows
+// (grid.y) fills CUs that linear_mt, a block per 16 weight rows, would leave idle; the
+// repeated reads of so small a W come from the caches.
+//   * Up to one such tile per CU.
+//   * Plain stages of more than 32 rows whose X is row-major, up to two per CU (4
+//     waves each): linear_mt's X loads are 64-byte pieces there.  With packed X it is
+//     the faster one (VL-2B layer at 48 rows 71.5 against 75.5 us).
+//   * SwiGLU of K <= 1024 (a chunk per wave), up to two per CU.
+// Measured, us, linear_mt / tiles at 17, 32, 64 rows: Qwen3-0.6B o_proj 6.4 / 5.6, 7.8
+// / 5.5, 11.8 / 5.6, down 8.0 / 7.5, 10.0 / 7.6, 15.9 / 7.7; VL-2B o_proj 6.7 / 5.9,
+// 8.0 / 5.9, 12.2 / 8.6, down 13.4 / 12.8, 17.5 / 12.7, 28.6 / 22.0 (row-major X); on
+// the other side of the line Qwen3-8B o_proj 11.2 / 15.5, 14.4 / 17.4, 21.8 / 33.0.
+template <bool SILU>
+bool narrow(const LinearArgs& a) {
+  const int64_t cus = num_cus(), gy = (a.M + 15) / 16, tiles = (a.N + 15) / 16 * gy;
+  const bool two = SILU ? a.K <= 1024 : (gy > 2 && !a.x_packed);
+  return tiles <= (two ? 2 * cus : cus);
+}
+
+// M > 4.  Up to 16 rows SwiGLU and two shapes of the plain stages, and above them
+// narrow matrices, keep the 16-row kernels; everything else runs linear_mt (its own X
+// extents permitting).
 template <bool SILU>
 void launch_mfma(const LinearArgs& a, hipStream_t s) {
-  const int64_t tx = (a.N + 15) / 16, cus = num_cus();
+  const int64_t tx = (a.N + 15) / 16, tiles = tx * ((a.M + 15) / 16), cus = num_cus();
   const int64_t nchunks = (a.K + kMfmaKC - 1) / kMfmaKC;
-  const bool mt = linear_mt_supported(a);
-  if (a.M > 16 && mt) return launch_linear_mt(a, s);
+  const bool mt = linear_mt_supported(a), few = a.M > 16 && narrow<SILU>(a);
+  if (a.M > 16 && mt && !few) return launch_linear_mt(a, s);
   if constexpr (SILU) {
     // gate/up of the model shapes (K = 4096: 4 chunks per wave): 3 or 2
     // tiles per CU run as multi-tile blocks, one per CU.
@@ -1130,39 +1147,42 @@ void launch_mfma(const LinearArgs& a, hipStream_t s) {
       else hipLaunchKernelGGL((linear_mfma_kernel<2, true, 4, 4, 2>), grid, block, 0, s, a);
       return;
     }
-    launch_mfma_tiles<true>(a, s);
+    launch_mfma_nw<true, 4>(a, s);
   } else {
     // 16 < rows per CU <= 24 (QKV of the model: 6144 rows, 24 per CU): one
     // 24-row block per CU instead of 16-row tiles two to some CUs.
     if (a.M <= 16 && a.N > 16 * cus && a.N <= 24 * cus) launch_mfma_r2<8>(a, s);
     else if (tx >= 4 * cus && nchunks == 16 && a.K % kMfmaKC == 0) launch_mfma_stream(a, cus, s);
-    else if (mt) launch_linear_mt(a, s);
-    else launch_mfma_tiles<false>(a, s);
+    else if (mt && !few) launch_linear_mt(a, s);
+    else if (tiles > cus && tiles <= 2 * cus) launch_mfma_nw<false, 4>(a, s);  // two 68 KB blocks to a CU
+    else launch_mfma_nw<false, 8>(a, s);
   }
 }
 
-// The batched stages with the RMSNorm prologue (4 < M <= 16, K = 4096: four
-// 256-wide chunks per wave) run the X-stationary kernel, which normalises in
-// its prologue: gate/up with 2 or 3 tiles per CU as multi-tile blocks, the
-// 24-row blocks of a QKV-sized projection, and up to one 16-row tile per CU.
-// Larger shapes (an LM head) keep the staging pass and the streaming blocks.
+// The batched stages with the RMSNorm prologue (M > 4, K = 4096: four 256-wide
+// chunks per wave) run the X-stationary kernel, which normalises in its
+// prologue: up to 16 batch rows gate/up with 2 or 3 tiles per CU as multi-tile
+// blocks and the 24-row blocks of a QKV-sized projection, and up to one tile of 16
+// weight rows by 16 batch rows per CU.  Larger shapes (an LM head) keep the
+// staging pass and the streaming blocks.
 bool launch_xs_norm(const LinearArgs& a, hipStream_t s) {
-  if (a.M > 16 || a.K != 4 * 4 * kMfmaKC || a.x_packed) return false;
+  if (a.K != 4 * 4 * kMfmaKC || a.x_packed) return false;
   const int64_t cus = num_cus(), tx = (a.N + 15) / 16;
+  const unsigned gy = unsigned((a.M + 15) / 16);
   const dim3 block(4 * kWave);
   if (a.epi == kEpiSilu) {
-    if (tx == 3 * cus) hipLaunchKernelGGL((linear_xs_kernel<2, true, 4, 3, 0, true>), dim3(unsigned(cus)), block, 0, s, a);
-    else if (tx == 2 * cus) hipLaunchKernelGGL((linear_xs_kernel<2, true, 4, 2, 0, true>), dim3(unsigned(cus)), block, 0, s, a);
-    else if (tx <= cus) hipLaunchKernelGGL((linear_xs_kernel<2, true, 4, 1, 0, true>), dim3(unsigned(tx)), block, 0, s, a);
+    if (gy == 1 && tx == 3 * cus) hipLaunchKernelGGL((linear_xs_kernel<2, true, 4, 3, 0, true>), dim3(unsigned(cus)), block, 0, s, a);
+    else if (gy == 1 && tx == 2 * cus) hipLaunchKernelGGL((linear_xs_kernel<2, true, 4, 2, 0, true>), dim3(unsigned(cus)), block, 0, s, a);
+    else if (tx * gy <= cus) hipLaunchKernelGGL((linear_xs_kernel<2, true, 4, 1, 0, true>), dim3(unsigned(tx), gy), block, 0, s, a);
     else return false;
     return true;
   }
-  if (a.N > 16 * cus && a.N <= 24 * cus) {
+  if (gy == 1 && a.N > 16 * cus && a.N <= 24 * cus) {
     hipLaunchKernelGGL((linear_xs_kernel<2, false, 4, 1, 8, true>), dim3(unsigned((a.N + 23) / 24)), block, 0, s, a);
     return true;
   }
-  if (tx <= cus) {
-    hipLaunchKernelGGL((linear_xs_kernel<1, false, 4, 1, 0, true>), dim3(unsigned(tx)), block, 0, s, a);
+  if (tx * gy <= cus) {
+    hipLaunchKernelGGL((linear_xs_kernel<1, false, 4, 1, 0, true>), dim3(unsigned(tx), gy), block, 0, s, a);
     return true;
   }
   return false;
@@ -1200,8 +1220,8 @@ int launch_linear(const LinearArgs& a, hipStream_t s) {
       silu ? launch_valu_m<false, true>(a, s) : launch_valu_m<false, false>(a, s);
     }
   } else {
-    // 4 < M <= 16 with the RMSNorm prologue: the X-stationary kernel normalises
-    // in its prologue where the shape allows (one block per CU: every block
+    // M > 4 with the RMSNorm prologue: the X-stationary kernel normalises in its
+    // prologue where the shape allows (one block per CU: every block
     // loads X once anyway); otherwise the input is staged once as
     // bf16(x * rsqrt(mean x^2 + eps) * w) (the reference's staging) into the
     // caller's workspace and a plain MFMA GEMM runs on it (normalising inside

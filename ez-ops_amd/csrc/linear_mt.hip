@@ -5,7 +5,9 @@
 // 64 rows the projections took four times their weight traffic.  Here a block
 // owns 16 weight rows (T = 2: 16 + 16, the gate and up rows of SwiGLU or two
 // neighbouring tiles) against MT 16-row batch blocks: each weight fragment is
-// read from LDS once and meets MT activation fragments.
+// read from LDS once and meets MT activation fragments.  (Matrices with too few
+// 16-row tiles to fill the chip this way stay with the 16-row kernels: narrow() in
+// gemv.hip.)
 //
 //   * 4 waves split K into 256-wide chunks; a chunk of a 16-row tile (8 KiB)
 //     lands in LDS by DMA (buffer_load_dwordx4 ... lds) in 512-byte row pieces

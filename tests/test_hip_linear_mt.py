@@ -1,6 +1,8 @@
-"""Linear stages of 5 and more batch rows (one read of W per 64 rows) against the oracle.
+"""Linear stages of 5 and more batch rows against the oracle, on both sides of the line
+between the tiles of 16 by 16 rows (above 16 batch rows: matrices of few weight
+rows) and the kernel that reads W once per 64 rows.
 
-Sizes at the edges of the kernel: batch blocks of 16 (1 to 4 per block,
+Sizes at the edges of the kernels: batch blocks of 16 (1 to 4 per block,
 two 64-row groups), weight-row remainders of a 16-row tile, K with fewer
 chunks than waves and a masked last chunk, one tile per CU / two blocks per
 CU / two-tile blocks.  Bar: bf16 allclose(atol 2e-2, rtol 1e-2) against the
@@ -54,6 +56,30 @@ def _run(M, N, K, epi, norm, pad=0, seed=0):
 @pytest.mark.parametrize("N,K", [(48, 512), (37, 1032), (16, 40), (250, 2048)])
 def test_linear_mt_edges(M, epi, norm, N, K):
     _run(M, N, K, epi, norm, pad=0 if norm else 8 * (N % 2))
+
+
+# the same edges where the matrix is wide enough for one read of W per 64 rows
+@pytest.mark.parametrize("M", [17, 32, 33, 48, 49, 64, 65, 96, 97, 100])
+@pytest.mark.parametrize("epi,norm", [(0, 0), (1, 0), (2, 1), (3, 0)])
+@pytest.mark.parametrize("N,K", [(4133, 40), (4112, 1032)])
+def test_linear_mt_edges_wide(M, epi, norm, N, K):
+    _run(M, N, K, epi, norm, pad=0 if norm else 8 * (N % 2))
+
+
+def _tiles(n):
+    """Weight rows of n 16-row tiles, n in tiles per CU."""
+    return 16 * int(n * torch.cuda.get_device_properties(0).multi_processor_count)
+
+
+# the line itself: (tiles per CU of the matrix, batch rows) with the last shape of the 16 x 16 tiles and the first
+# beyond it -- one tile per CU; two for plain stages of more than 32 rows and for SwiGLU of K <= 1024; the norm
+# inside the kernel (K = 4096) up to one
+@pytest.mark.parametrize("over", [0, 16])
+@pytest.mark.parametrize("tiles,M,K,epi,norm", [(1 / 2, 32, 512, 1, 0), (1 / 2, 64, 256, 1, 0), (1 / 4, 64, 768, 0, 1),
+                                                (1 / 4, 64, 4096, 0, 1), (1 / 2, 20, 4096, 2, 1), (1 / 4, 64, 2048, 2, 1),
+                                                (1 / 2, 64, 1024, 2, 1), (1 / 4, 128, 512, 3, 0)])
+def test_linear_narrow_line(tiles, M, K, epi, norm, over):
+    _run(M, _tiles(tiles) + over, K, epi, norm, seed=2)
 
 
 # 4104 rows: two blocks per CU and a remainder; 5200 and 16400: two-tile blocks,
