@@ -325,12 +325,15 @@ void launch_m(const LinearArgs& a, bool vec, hipStream_t s) {
 }  // namespace
 
 // M > 4, operands checked by launch_linear (16-byte rows, 32-bit extents).
+// 65 to 96 rows go in two equal groups, not 64 and the rest: 0.6B gate/up 16.5 -> 15.2 us at
+// 65 rows (13.9 with 16 rows per read of W), VL-2B o_proj 12.0 -> 10.0 (11.3), o_proj + FFN 0.6B
+// 33.4 -> 31.2 (31.8), VL-2B 58 -> 52.
 void launch_linear_mt(const LinearArgs& a, hipStream_t s) {
   const bool vec = a.ldy % 4 == 0 && (reinterpret_cast<uintptr_t>(a.Y) & 7) == 0 &&
                    (a.epi != kEpiResid || (a.ldr % 4 == 0 && (reinterpret_cast<uintptr_t>(a.res) & 7) == 0));
   if (a.M <= 16) launch_m<1>(a, vec, s);
   else if (a.M <= 32) launch_m<2>(a, vec, s);
-  else if (a.M <= 48) launch_m<3>(a, vec, s);
+  else if (a.M <= 48 || (a.M > 64 && a.M <= 96)) launch_m<3>(a, vec, s);
   else launch_m<4>(a, vec, s);
 }
 
