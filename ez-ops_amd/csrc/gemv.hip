@@ -1013,13 +1013,15 @@ void launch_rows_t(const LinearArgs& a, hipStream_t s) {
   // ramp: one batch row, <= 1024 blocks of four rows: one row (GEMV 4096 x 4096,
   // 4 / 2 / 1 rows: 8.0 / 7.7 / 7.5 us; two rows at K = 6144 and 2048 rows, 1024
   // or 2048 blocks: 6.20 / 6.24 us).  Two to four: below 1024 blocks of four
-  // rows one row (K <= 4096) or two (4096 x 4096 at batch 4, 4 / 2 / 1 rows: 9.1 /
-  // 10.0 / 12.8 us; 2048 x 2048: 5.1 / 4.7 / 4.7); with the prologue, below 512
+  // rows (one full chunk a thread: up to 1024) one row (K <= 4096) or two (4096 x 4096
+  // at batch 4, 4 / 2 / 1 rows: 9.1 / 10.0 / 12.8 us; 2048 x 2048: 5.1 / 4.7 / 4.7; four
+  // and one at batch 2 and 4: 4096 x 2048 5.33 / 4.9, 6.3 / 5.9; 4096 x 1536, a masked
+  // chunk, 4.7 / 5.4, 5.8 / 6.2); with the prologue, below 512
   // blocks half the rows (Qwen3-0.6B QKV at batch 4, 8 / 4 / 1: 6.4 / 5.9 / 8.3).
   if constexpr (M > 1 && NORM) {
     if (blocks < 512 && RB > 1) return launch(std::integral_constant<int, (RB > 1 ? RB / 2 : 1)>{});
   } else if constexpr (M > 1 && !SILU && RB == 4) {
-    if (blocks < 1024) return launch(std::integral_constant<int, (CH <= 2 ? 1 : 2)>{});
+    if (blocks < 1024 + (CH == 1 && !TAIL)) return launch(std::integral_constant<int, (CH <= 2 ? 1 : 2)>{});
   } else if constexpr (M == 1 && RB == 4) {
     if (blocks <= 1024) return launch(std::integral_constant<int, 1>{});
   }
