@@ -43,3 +43,23 @@ def test_paged_attn_decode_plan_zero_length():
     want = gqa_decode_reference(Q, paged_to_contiguous(Kp, bt), paged_to_contiguous(Vp, bt), lens.clamp(min=1))
     torch.testing.assert_close(out[live].float(), want[live].float(), rtol=1e-2, atol=1e-2)
     assert (out[5] == 0).all()
+
+
+# more sequences than a block's length scan holds (64): equal splits of the longest for every sequence
+@pytest.mark.parametrize("B,H,Hkv,D,S", [(65, 32, 8, 128, 600), (65, 8, 8, 128, 1024), (80, 16, 8, 64, 2080),
+                                         (100, 16, 1, 128, 1536), (130, 4, 2, 128, 1040)])
+@pytest.mark.parametrize("long", [0, 64])
+def test_attn_decode_many_sequences(B, H, Hkv, D, S, long):
+    """One long sequence among short ones (an empty one too): every split but the long sequence's first is empty."""
+    g = torch.Generator(device="cuda").manual_seed(B + S)
+    r = lambda *s: torch.randn(*s, generator=g, device="cuda").to(torch.bfloat16)  # noqa: E731
+    Q, K, V = r(B, H, 1, D), r(B, Hkv, S, D), r(B, Hkv, S, D)
+    lens = torch.randint(1, 40, (B,), generator=g, device="cuda").to(torch.int32)
+    lens[long], lens[5] = S, 0
+    for b, n in enumerate(lens.tolist()):
+        K[b, :, n:], V[b, :, n:] = float("nan"), float("nan")
+    out = AttnDecodeOp(B, H, S, D, "hip", Hkv)(Q, K, V, lens)
+    want = gqa_decode_reference(Q, K.nan_to_num(0.0), V.nan_to_num(0.0), lens.clamp(min=1))
+    live = lens.long() > 0
+    torch.testing.assert_close(out[live].float(), want[live].float(), rtol=1e-2, atol=1e-2)
+    assert (out[5] == 0).all()

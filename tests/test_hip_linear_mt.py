@@ -88,3 +88,33 @@ def test_linear_narrow_line(tiles, M, K, epi, norm, over):
                                             (64, 4096, 4096, 1, 0), (40, 4112, 1024, 2, 1)])
 def test_linear_mt_tilings(M, N, K, epi, norm):
     _run(M, N, K, epi, norm, seed=1)
+
+
+# per_cu: 16-row weight tiles per CU -- the streaming, multi-tile and one-tile launches
+@pytest.mark.parametrize("per_cu,K,epi", [(4, 4096, 0), (3, 512, 1), (3, 4096, 2), (2, 4096, 2), (1, 520, 2), (1 / 4, 40, 3)])
+def test_linear_rows_far_apart(per_cu, K, epi):
+    """20 batch rows at a stride of 2^23 elements and more, beyond the 32-bit extents of a 64-row block of X: two batch
+    blocks of the 16-row kernels.  Against fp32 torch on the same GPU, the bar above."""
+    M, N, ldx = 20, _tiles(per_cu) + 8, (1 << 23) + 8
+    if per_cu in (2, 3):
+        N -= 8  # the multi-tile launches need whole tiles
+    gen = torch.Generator(device=DEV).manual_seed(N + K)
+    r = lambda *s: torch.randn(*s, generator=gen, device=DEV).to(torch.bfloat16)  # noqa: E731
+    buf = torch.zeros(M * ldx, dtype=torch.bfloat16, device=DEV)
+    X = buf.view(M, ldx)[:, :K]
+    X.copy_(r(M, K))
+    W, W2, R = r(N, K) * 2.0 ** -6, r(N, K) * 2.0 ** -6, r(M, N)
+    Xf = X.float()
+    ref = Xf @ W.float().T
+    if epi != 3:
+        ref = ref.bfloat16().float()
+    if epi == 1:
+        ref = (R.float() + ref).bfloat16().float()
+    elif epi == 2:
+        ref = torch.nn.functional.silu(ref).bfloat16().float() * (Xf @ W2.float().T).bfloat16().float()
+    Y = torch.full((M + 1, N), 7.0, dtype=torch.float32 if epi == 3 else torch.bfloat16, device=DEV)
+    _hip.call("ezops_linear_stage_bf16", X.data_ptr(), ldx, W.data_ptr(), W2.data_ptr(), Y.data_ptr(), N, R.data_ptr(), N,
+              None, 0, 1e-6, epi, M, N, K, None, 0, _hip.stream())
+    torch.cuda.synchronize()
+    assert (Y[M] == 7.0).all()
+    torch.testing.assert_close(Y[:M].float(), ref, rtol=1e-2, atol=2e-2)

@@ -392,12 +392,13 @@ def test_gemv_rows_widths(M, K, epi, norm):
     np.testing.assert_allclose(n(Y), ref, **BF_TOL)
 
 
-@pytest.mark.parametrize("M,N", [(16, 12288), (20, 8192), (8, 12288)])
-def test_linear_stage_swiglu_multi_tile(M, N):
-    """Gate/up shapes whose 16-row tiles are 3x / 2x the CU count run as
-    multi-tile blocks (the DMA ring continues across tiles): bit-exact with
-    the one-tile-per-block launch on the same rows, and against the oracle."""
-    K = 4096
+@pytest.mark.parametrize("M,per_cu", [(16, 3), (8, 3), (16, 2), (5, 2)])
+def test_linear_stage_swiglu_multi_tile(M, per_cu):
+    """Gate/up shapes of up to 16 rows whose 16-row tiles are 3x / 2x the CU
+    count run as multi-tile blocks (the DMA ring continues across tiles):
+    bit-exact with the one-tile-per-block launch on the same rows, and against
+    the oracle."""
+    N, K = 16 * per_cu * torch.cuda.get_device_properties(0).multi_processor_count, 4096
     rng = np.random.default_rng(M + N)
     X = oracle.bf16(rng.standard_normal((M, K)).astype(np.float32))
     W = oracle.bf16(rng.standard_normal((N, K)).astype(np.float32) * K ** -0.5)
@@ -427,7 +428,7 @@ def test_linear_stage_24_row_blocks(M, extra, K, epi):
     CUs) runs one block of 16 + 8 rows per CU, the two MFMA tiles sharing
     each X fragment; N = 16 * CUs + extra covers the full case (extra =
     8 * CUs), a partial last block and a block whose second tile is empty.
-    M = 20 takes the 16-row tiles (two batch blocks) for comparison."""
+    M = 20 takes the kernel that reads W once per 64 rows, for comparison."""
     cus = torch.cuda.get_device_properties(0).multi_processor_count
     N = 16 * cus + (extra if extra < 2048 else 8 * cus)
     rng = np.random.default_rng(M + N + K + epi)
@@ -451,8 +452,9 @@ def test_linear_stage_24_row_blocks(M, extra, K, epi):
 @pytest.mark.parametrize("M,extra,epi", [(16, 37, 0), (5, 0, 1), (20, 1000, 3), (16, 8192, 1)])
 def test_linear_stage_streaming_blocks(M, extra, epi):
     """At least four 16-row tiles per CU and K = 4096 (an LM head at batch
-    > 4): two streaming blocks per CU walk the tiles with one DMA ring;
-    ragged last tiles, partial batch blocks and every store form."""
+    5 to 16): two streaming blocks per CU walk the tiles with one DMA ring;
+    ragged last tiles, partial batch blocks and every store form.  M = 20
+    takes the kernel that reads W once per 64 rows."""
     cus = torch.cuda.get_device_properties(0).multi_processor_count
     N, K = 4 * 16 * cus + extra, 4096
     rng = np.random.default_rng(M + N + epi)
@@ -479,8 +481,9 @@ def test_linear_stage_streaming_blocks(M, extra, epi):
 def test_linear_stage_norm_in_kernel(M, shape):
     """Batched stages with the RMSNorm prologue at K = 4096 normalise inside
     the X-stationary kernel (no staging pass): gate/up with 3 and 2 tiles per
-    CU (multi-tile blocks), the 24-row QKV blocks, and a few 16-row tiles;
-    M = 20 spans two batch blocks (multi-tile and one-tile shapes)."""
+    CU (multi-tile blocks), the 24-row QKV blocks, and a few 16-row tiles.
+    M = 20 spans two batch blocks in the one-tile shapes; its gate/up shapes
+    take the staging pass and the kernel that reads W once per 64 rows."""
     cus = torch.cuda.get_device_properties(0).multi_processor_count
     K = 4096
     N, epi = {"gate_up3": (48 * cus, 2), "gate_up2": (32 * cus, 2), "qkv24": (24 * cus, 0), "tiles": (200, 1)}[shape]
