@@ -112,8 +112,8 @@ __global__ __launch_bounds__(kGThreads, WPE) void gemm_bf16_kernel(GemmArgs a) {
   constexpr int kRowBytes = BK * 2, kSub = BK / 16;        // MFMA substeps per K-step
   constexpr int kXBytes = BM * kRowBytes, kWBytes = BN * kRowBytes;
   EZ_PROF_WAVE(kProfGemm);
-  // Two stages of X tiles and three of W tiles (160 KiB at 256 x 256); after the
-  // K loop the same memory holds the block's C tile in bf16, wave by wave, for
+  // SX stages of X tiles and SW of W tiles (256 x 256: two and three, 160 KiB); after
+  // the K loop the same memory holds the block's C tile in bf16, wave by wave, for
   // row-contiguous stores.
   __shared__ __align__(16) uint16_t lds[(SX * BM + SW * BN) * BK];
 
@@ -442,6 +442,11 @@ int gemm_bf16(const uint16_t* X, int64_t ldx, const uint16_t* W, uint16_t* Y, in
 }  // namespace ez
 
 extern "C" size_t ezops_gemm_workspace_size(void) { return 0; }
+
+extern "C" int ezops_gemm_tile(int64_t M, int64_t N, int swiglu, int64_t cus) {
+  EZ_REQUIRE(M >= 1 && N >= 1 && cus >= 1, "gemm_tile: sizes must be >= 1");
+  return ez::pick_tile(M, N, swiglu != 0, cus);
+}
 
 extern "C" int ezops_gemm_swiglu_bf16(const void* X, int64_t ldx, const void* Wgu, void* Y, int64_t ldy, int64_t M,
                                       int64_t IS, int64_t K, hipStream_t stream) {

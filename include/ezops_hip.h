@@ -301,6 +301,12 @@ int ezops_gemm_bf16(const void* X, int64_t ldx, const void* W, void* Y, int64_t 
                     int64_t M, int64_t N, int64_t K, void* workspace, size_t workspace_bytes,
                     hipStream_t stream);
 
+/* The tile shape ezops_gemm_bf16 (swiglu = 0; N = columns of Y) or
+ * ezops_gemm_swiglu_bf16 (swiglu = 1; N = 2 IS) takes for an [M, N] product on
+ * `cus` CUs: the index into the tile table of gemm.hip, or EZOPS_EINVAL.  Host
+ * only; for tests and profiles.  No counterpart in the reference. */
+int ezops_gemm_tile(int64_t M, int64_t N, int swiglu, int64_t cus);
+
 /* Prefill gate/up projection fused with SwiGLU:
  * Y[M, IS] = bf16(bf16(silu(bf16(X Wg^T))) * bf16(X Wu^T)) with Wgu = [Wg; Wu]
  * as [2 IS, K] (the layer's gate/up weight), bit-identical to

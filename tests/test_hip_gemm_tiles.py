@@ -1,6 +1,7 @@
 """Prefill GEMM at every tile shape's edges (GPU): row, column and K remainders,
 fewer K-steps than pipeline stages, and the same rows bit-identical whichever
-shape serves them.  Bar: bf16 allclose(atol 2e-2, rtol 1e-2) of the fp32 product
+shape serves them; that the sizes reach every tile shape is checked on the CPU.
+Bar: bf16 allclose(atol 2e-2, rtol 1e-2) of the fp32 product
 (W of exact powers scaled so that outputs are O(1))."""
 
 import pytest
@@ -8,7 +9,7 @@ import torch
 
 from ezops import _hip
 
-pytestmark = pytest.mark.gpu
+gpu = pytest.mark.gpu
 DEV = "cuda"
 
 
@@ -29,13 +30,31 @@ def _data(M, N, K, seed=0):
     return X, W
 
 
-# (M, N) chosen so that, on 256 CUs, each tile shape of the table is picked:
-# 256x256, 256x192, 256x128, 128x128 (two per CU), 128x128 (K-steps of 128), 64x128
-# (three times), 192x256
+CUS = 256  # MI355X
+# (M, N) chosen so that each tile shape of the table is picked: 256x256, 256x192, 256x128,
+# 128x128 (two per CU), 128x128 (K-steps of 128), 64x128 (three times), 192x256
 SHAPES = [(4000, 4090), (2040, 6136), (2040, 4090), (700, 6136), (1020, 4090), (200, 6136), (1, 130), (65, 72),
           (3000, 4090)]
+# gate/up (M, IS): 256x256, 192x256, 256x256, 128x128 (two per CU), 128x128 (K-steps of 128, three
+# times), 256x128 twice
+SWIGLU_SHAPES = [(500, 12288), (740, 12288), (4000, 2048), (600, 12288), (120, 12288), (1, 128), (130, 384), (499, 6144),
+                 (1000, 3072)]
 
 
+def _tile(M, N, swiglu):
+    return _hip.lib().ezops_gemm_tile(M, N, swiglu, CUS)
+
+
+@pytest.mark.parametrize("swiglu", [0, 1])
+def test_shapes_reach_every_tile(swiglu):
+    """Every tile shape the rule picks anywhere in a sweep of prompt lengths and projection sizes is one that a size
+    below picks (CPU)."""
+    tested = {_tile(M, 2 * N if swiglu else N, swiglu) for M, N in (SWIGLU_SHAPES if swiglu else SHAPES)}
+    picked = {_tile(M, N, swiglu) for M in range(1, 6000, 37) for N in range(256, 26000, 256)}
+    assert picked <= tested and len(tested) == (5 if swiglu else 7)
+
+
+@gpu
 @pytest.mark.parametrize("M,N", SHAPES)
 @pytest.mark.parametrize("K", [8, 72, 128, 192, 264, 520, 1032])
 @pytest.mark.parametrize("resid", [False, True])
@@ -48,6 +67,7 @@ def test_gemm_tile_edges(M, N, K, resid):
     torch.testing.assert_close(_gemm(X, W, R).float(), ref, rtol=1e-2, atol=2e-2)
 
 
+@gpu
 @pytest.mark.parametrize("K", [520, 4096])
 def test_gemm_tile_shapes_bit_identical(K):
     X, W = _data(4000, 6136, K, seed=1)
@@ -56,8 +76,8 @@ def test_gemm_tile_shapes_bit_identical(K):
         assert torch.equal(_gemm(X[:M], W[:N]), full[:M, :N]), (M, N)
 
 
-# gate/up: 256x256 twice, 128x128 (two per CU), 192x256, 128x128
-@pytest.mark.parametrize("M,IS", [(500, 12288), (740, 12288), (4000, 2048), (600, 12288), (120, 12288), (1, 128), (130, 384)])
+@gpu
+@pytest.mark.parametrize("M,IS", SWIGLU_SHAPES)
 @pytest.mark.parametrize("K", [40, 128, 520])
 def test_gemm_swiglu_tiles_match_plain(M, IS, K):
     X, W = _data(M, 2 * IS, K, seed=2)
