@@ -89,3 +89,33 @@ def test_wide_matrices(M, N, K, epi, norm):
         ref = torch.nn.functional.silu(ref).to(BF).float() * (Xn @ W2.float().T).to(BF).float()
     got = _stage(X, W, epi, norm, W2, R, w).float()
     torch.testing.assert_close(got, ref, rtol=1e-2, atol=2e-2)
+
+
+def test_bf16_rounding_of_every_exponent():
+    """fp32 results rounded to bf16 (to nearest even) over all exponents, subnormal ones, ties, the largest values and
+    NaN, bit for bit as torch rounds them.  A result is the exact sum of three bf16 parts, scaled by 2^60 in W and back
+    in X below 2^-60 so that the parts are normal numbers."""
+    gen = torch.Generator().manual_seed(0)
+    bits = torch.randint(0, 1 << 32, (8192,), generator=gen)
+    bits[:2048] = bits[:2048] & ~0xffff | 0x8000  # ties
+    bits[2048:3072] = bits[2048:3072] & 0x80ffffff  # subnormal, and the smallest normal numbers
+    bits[3072:3200] = bits[3072:3200] & 0x8000ffff | 0x7f7f0000  # about the largest bf16: to it or to infinity
+    v = torch.where(bits >= 1 << 31, bits - (1 << 32), bits).to(torch.int32).view(torch.float32)
+    v = v[torch.isfinite(v)]
+    small = v.abs() < 2.0 ** -60
+    u = torch.where(small, v.double() * 2.0 ** 60, v.double())
+    trunc = lambda x: (x.float().view(torch.int32) & -65536).view(torch.float32).double()  # noqa: E731
+    hi = trunc(u)
+    mid = trunc(u - hi)
+    lo = u - hi - mid
+    assert (trunc(lo) == lo).all()
+    for sel, scale in ((~small, 1.0), (small, 2.0 ** -60)):
+        W = torch.zeros(int(sel.sum()), 8, dtype=BF, device=DEV)
+        for j, part in enumerate((hi, mid, lo)):
+            W[:, j] = part[sel].to(BF).to(DEV)
+        X = torch.zeros(1, 8, dtype=BF, device=DEV)
+        X[0, :3] = scale
+        got = _stage(X, W, 0)[0].cpu()
+        assert torch.equal(got.view(torch.int16), v[sel].to(BF).view(torch.int16))
+    nan = _stage(torch.ones(1, 8, dtype=BF, device=DEV), torch.full((1, 8), NAN, dtype=BF, device=DEV), 0)
+    assert torch.isnan(nan).all()
