@@ -303,8 +303,10 @@ __global__ __launch_bounds__(W * kWave) void attn_split_kernel(AttnArgs a, int n
     // (sequence, kv head, split) order; blocks past the active ones leave
     // before loading anything.  Lane j < B holds sequence j's length, and a
     // wave scan its first block.  (Ordering the sequences longest first cost
-    // ~1000 instructions per block before its first load and balanced nothing:
-    // a block's share is between half a chunk and a chunk whatever its length.
+    // ~1000 instructions per block before its first load and balanced little: a
+    // block's share is at most one chunk (rounded up to its waves' tiles), more
+    // than half of one in a sequence longer than a chunk, and the whole length
+    // of a shorter one.
     // Qwen3-8B layer, 64 ragged sequences up to 4096 rows, paged: attention 122.6
     // -> 97 us; 16 up to 16384: 85.5 -> 81.)
     const int B = int(a.B);
@@ -703,7 +705,9 @@ SplitPlan plan_splits(int64_t B, int64_t Hkv, int64_t Lh, int64_t G, bool balanc
   if (waves == 4 && balance) {
     // Beyond one block for each of the two places on a CU, a split keeps at
     // least 512 rows: four tiles per wave to carry the block's prologue and
-    // merge.  (Qwen3-8B layer's attention, 64 sequences of 512 rows: one split
+    // merge.  Also above 64 sequences, where every sequence gets the same splits: 65-192
+    // sequences, group sizes 1-16, both head sizes, full, ragged or one long among short
+    // ones, 0.95-1.95 of the time without it.  (Qwen3-8B layer's attention, 64 sequences of 512 rows: one split
     // 27.8 us, four and a merge launch 63.4 + 4.9; 32 ragged sequences up to 1024
     // rows 18.9 against 38.0; at least 256 rows: 27.1 + 4.8 and 22.0.)
     const int64_t fill = (2 * cus + units - 1) / units, rows = Lh / 512;

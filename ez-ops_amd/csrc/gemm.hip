@@ -32,11 +32,14 @@
 // while they could still be read: gate/up at 4096 tokens 683 -> 650 us, QKV
 // 201 -> 192, o_proj 136 -> 126, down 331 -> 316; same run).
 //
-// What bounds it: every shape moves about 115 bytes of LDS traffic (fragment
-// reads + DMA writes) per clock and CU, close to the LDS's 128; 256 x 256 needs
-// 256 KiB of it per step, as many cycles as its MFMAs.  Small tiles need more
-// per flop but fill the chip at short prompts; their K-steps of 128 halve the
-// barriers and the scalar work per K (128 x 128 at K = 4096: 38 -> 29 us).
+// What bounds it: LDS traffic (fragment reads + DMA writes) beside the MFMAs at the
+// clock that this load leaves.  Counters at 4096 tokens, Qwen3-8B's gate/up, down,
+// QKV, o_proj: 106, 104, 112 and 87 bytes per clock and CU of the LDS's 128, matrix
+// cores busy 80, 79, 73 and 63% of the cycles, at 1.6-1.8 GHz.  256 x 256 needs 256
+// KiB per step, as many cycles as its MFMAs.  Small tiles need more per flop but fill
+// the chip at short prompts (740 tokens: 70-82 bytes per clock, a part-filled round);
+// their K-steps of 128 halve the barriers and the scalar work per K (128 x 128 at K =
+// 4096: 38 -> 29 us).
 //
 // Rows are stored with their 16-byte chunks XOR-swizzled (by (row >> 1) & 7, or
 // row & 15 for 256-byte rows): gfx950's LDS is 64 banks (256 bytes) wide, and a

@@ -737,7 +737,11 @@ __global__ __launch_bounds__(4 * kWave) void linear_xs_kernel(LinearArgs a) {
 // instruction straight from the packed pairs (v_dot2_f32_bf16): from two batch
 // rows on the kernel is bound by its arithmetic (gate/up at batch 4 46.8 -> 41.5
 // us, down 25.7 -> 23.2).  Otherwise unpacked FMAs, which a single batch row
-// hides under its loads.
+// hides under its loads.  The pair's products and c are added with one rounding;
+// subnormal operands, products and sums are kept, as by the FMAs.  Errors
+// of fp32 results against fp64, rms, FMA / DOT2 at batch 2: K = 256 5.59e-8 / 5.60e-8 of
+// the results' rms, 4096 7.89 / 7.85, 16384 9.24 / 9.07.  The one difference: two
+// products of a pair beyond fp32 with opposite signs make NaN (the FMAs: an infinity).
 template <bool DOT2>
 __device__ __forceinline__ float dot8(const uint4& a, const uint4& b, float c) {
   if constexpr (DOT2) {

@@ -25,7 +25,7 @@
 // Bound: HBM (weights) up to 32 rows; at 64 the X fragments, MT / T times the
 // weight bytes through each CU's L1.  Measured (MI355X, Qwen3-8B, kernel
 // traces, this kernel against 16 rows per read of W): 64 rows: gate/up 45
-// against 131.7 us, QKV 18.7 / 38.1, o_proj + down 49 / 116.  32 rows: gate/up
+// against 131.7 us, QKV 17-18 / 38.1, o_proj + down 48 / 116.  32 rows: gate/up
 // 37.1, QKV 14.1 us (16 rows: 35.7, 15.6).  The X traffic costs about 1 us per
 // 18 MB over the chip; requesting X a whole chunk ahead (two chunks in
 // registers) changed nothing.  Up to 16 rows: VL-2B QKV + o_proj + down 24.4 ->
@@ -314,7 +314,7 @@ void launch_m(const LinearArgs& a, bool vec, hipStream_t s) {
   auto grid = [&](int64_t t, int64_t slots) { return unsigned(t < slots ? t : slots); };
   if (a.epi == kEpiSilu) return launch_x<2, true, MT>(a, grid(tiles, cus), vec, s);
   // Two-tile blocks (each X fragment meets 32 weight rows) where most CUs still
-  // have one: Qwen3-8B QKV (192 blocks) at 64 rows 22.1 -> 18.7 us, at 32 16.1 ->
+  // have one: Qwen3-8B QKV (192 blocks) at 64 rows 22.1 -> 17-18 us, at 32 16.1 ->
   // 14.1; o_proj and down on half the CUs lose (together 49 -> 59 us).
   if (4 * tiles > 5 * cus) return launch_x<2, false, MT>(a, grid((a.N + 31) / 32, cus), vec, s);
   // Else 16-row tiles, 4 waves each (8 waves splitting K: VL-2B QKV + o_proj +

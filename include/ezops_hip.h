@@ -49,7 +49,10 @@ int ezops_gemv_bf16(const void* A, const void* B, void* C, int64_t N, int64_t K,
 
 /* Skinny bf16 linear layer: Y[m, n] = sum_k X[m, k] * W[n, k] for m < M.
  * X [M, K] (row stride ldx), W [N, K], Y [M, N] (row stride ldy); M >= 1.
- * MFMA when M > 4, W read once per 64 rows.
+ * MFMA when M > 4; W read once per 64 rows (matrices too narrow to fill the
+ * chip that way: per 16).  Deterministic for given sizes; a row's last bits may
+ * differ between row counts of different kernels (1, 2-4, 5 and more), which sum
+ * over K in different orders.
  * Replaces: the `x @ W.T` projections inside the fused decode kernels
  * (ezops/kernels/fused_o_proj_ffn/fused_o_proj_ffn_triton.py:31-231,
  * ezops/kernels/qwen3_dense_decode/qwen3_dense_decode_triton.py:37-271). */
@@ -277,8 +280,11 @@ int ezops_qwen3_decode_step_bf16(const ezops_qwen3_layer* layers, int64_t n_laye
  * p->max_kv_len is unused.  block_table != NULL: paged caches as in
  * ezops_qwen3_dense_decode_paged_bf16.  max_q_len: host bound on the
  * per-sequence token counts.  D = 128, IS % 8 == 0.  The projections run
- * the library's own GEMM (see ezops_gemm_bf16): deterministic,
- * allocation-free and graph-capturable for every shape.
+ * the library's own GEMM (see ezops_gemm_bf16), in chunks of up to 64 tokens (HS
+ * <= 16384) the decode layer's linear stages: deterministic, allocation-free and
+ * graph-capturable for every shape.  Every tile shape of the GEMM gives a token
+ * the same bits; the linear stages sum over K in another order, so the last bits
+ * of a chunk of up to 64 tokens may differ from the same tokens' in a longer one.
  * No counterpart in the reference (decode only,
  * ezops/ops/qwen3_dense_decode.py:9-176): the step that fills the cache the
  * decode layer reads. */
